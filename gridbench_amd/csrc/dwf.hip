@@ -31,9 +31,9 @@
 
 namespace {
 
-// out = alpha * S x + beta * z, S = Mooee (INV false) or Mooee^-1 (INV true),
-// their adjoints for dag (chiralities exchanged).  z may be null (beta = 0).
-template <int P, bool INV>
+// out = alpha * Mooee x + beta * z, or the adjoint for dag (chiralities
+// exchanged).  z may be null (beta = 0).
+template <int P>
 __global__ void __launch_bounds__(256) k_dwf_s5(const void *x, void *out, const void *z, uint64_t ngroups,
                                                 uint32_t Ls, uint32_t nrhs, uint32_t gpw, double d_, double mass_,
                                                 double alpha_, double beta_, int dag)
@@ -45,9 +45,6 @@ __global__ void __launch_bounds__(256) k_dwf_s5(const void *x, void *out, const 
   const A d = (A)d_, mass = (A)mass_, alpha = (A)alpha_, beta = (A)beta_;
   const uint32_t lt = threadIdx.x, lg = lt / Ls, s = lt - lg * Ls;
   const bool in_group = lt < gpw * Ls;
-  A dinv = (A)1 / d, dls = (A)1;
-  for (uint32_t k = 0; k < Ls; k++) dls *= dinv;
-  const A gnorm = (A)1 / ((A)1 + mass * dls);  // 1 / (1 + mass d^-Ls)
   for (uint64_t g0 = (uint64_t)blockIdx.x * gpw; g0 < ngroups; g0 += (uint64_t)gridDim.x * gpw) {
     const uint64_t grp = g0 + lg;
     const bool active = in_group && grp < ngroups;
@@ -62,40 +59,104 @@ __global__ void __launch_bounds__(256) k_dwf_s5(const void *x, void *out, const 
       for (int j = 0; j < R; j++) {
         // P+ (reals 0..11) hops down in s (psi(s-1)), P- (12..23) up; dag exchanges them
         const bool down = ((kch * R + j) < 12) != (dag != 0);
-        A acc;
-        if (!INV) {
-          // d x(s) - x(s -/+ 1), the wrap replaced by +mass x(other end)
-          uint32_t sn;
-          A c;
-          if (down) {
-            sn = s == 0 ? Ls - 1 : s - 1;
-            c = s == 0 ? mass : (A)-1;
-          } else {
-            sn = s == Ls - 1 ? 0 : s + 1;
-            c = s == Ls - 1 ? mass : (A)-1;
-          }
-          acc = d * gx[(uint64_t)s * R + j] + c * gx[(uint64_t)sn * R + j];
+        // d x(s) - x(s -/+ 1), the wrap replaced by +mass x(other end)
+        uint32_t sn;
+        A c;
+        if (down) {
+          sn = s == 0 ? Ls - 1 : s - 1;
+          c = s == 0 ? mass : (A)-1;
         } else {
-          // sum_k d^-(k+1) L^k x: L^k x(s) = x(s -/+ k), times -mass once it wraps
-          acc = (A)0;
-          A w = dinv;
-          for (uint32_t k = 0; k < Ls; k++) {
-            uint32_t sk;
-            bool wrap;
-            if (down) {
-              wrap = k > s;
-              sk = wrap ? s + Ls - k : s - k;
-            } else {
-              wrap = s + k >= Ls;
-              sk = wrap ? s + k - Ls : s + k;
-            }
-            const A c = wrap ? -mass * w : w;
-            acc += c * gx[(uint64_t)sk * R + j];
-            w *= dinv;
-          }
-          acc *= gnorm;
+          sn = s == Ls - 1 ? 0 : s + 1;
+          c = s == Ls - 1 ? mass : (A)-1;
         }
+        const A acc = d * gx[(uint64_t)s * R + j] + c * gx[(uint64_t)sn * R + j];
         v[j] = alpha * acc;
+      }
+      if (z) {
+        A zv[R];
+        dev::load_chunk<P, A>(z, t, zv);
+#pragma unroll
+        for (int j = 0; j < R; j++) v[j] += beta * zv[j];
+      }
+      dev::store_chunk<P, A>(out, t, v, false);
+    }
+    __syncthreads();
+  }
+}
+
+// out = alpha * Mooee^-1 x + beta * z (dag: the adjoint), the sum
+// sum_k d^-(k+1) L^k x over the Ls slices of a group.
+//
+// Bound by memory (FP32 Ls16: 16 16-byte LDS reads and about 130 VALU
+// operations a 16-byte chunk, half the time its load and store take).  So
+// that the sum costs no more than that, a thread's Ls operands sit at fixed
+// offsets from one LDS address: a group is stored in the order its shift
+// walks it (position s, or Ls-1-s where L goes up in s) and twice over, so
+// L^k x is at position + Ls - k with no wrap to compute and one 16-byte read
+// holds every real of the chunk; only the coefficient looks at the wrap.  A
+// 16-bit chunk (8 reals, FP32 in LDS) is two such 4-real columns, since its
+// halves can differ in chirality.
+// 24^4 x Ls16 FP32: 684 us (1.5 TB/s; a wrapped address and a 4- or 8-byte
+// read per real and slice) -> 222 us (4.6 TB/s, a large copy reaches 4.85).
+template <int P>
+__global__ void __launch_bounds__(256) k_dwf_s5_inv(const void *x, void *out, const void *z, uint64_t ngroups, uint32_t Ls,
+                                                    uint32_t nrhs, uint32_t gpw, double d_, double mass_, double alpha_,
+                                                    double beta_, int dag)
+{
+  typedef typename dev::Traits<P>::acc A;
+  constexpr int R = dev::Traits<P>::R, NCH = dev::Traits<P>::NCH;
+  constexpr int SV = 16 / sizeof(A), H = R / SV;  // reals of an LDS entry, columns of a chunk
+  typedef A AV __attribute__((ext_vector_type(SV)));
+  extern __shared__ __align__(16) unsigned char smem[];
+  AV *sx = (AV *)smem;  // [gpw][H][2 * Ls]
+  const A d = (A)d_, mass = (A)mass_, alpha = (A)alpha_, beta = (A)beta_;
+  const uint32_t lt = threadIdx.x, lg = lt / Ls, s = lt - lg * Ls;
+  const bool in_group = lt < gpw * Ls;
+  A dinv = (A)1 / d, dls = (A)1;
+  for (uint32_t k = 0; k < Ls; k++) dls *= dinv;
+  const A gnorm = (A)1 / ((A)1 + mass * dls);  // 1 / (1 + mass d^-Ls)
+  for (uint64_t g0 = (uint64_t)blockIdx.x * gpw; g0 < ngroups; g0 += (uint64_t)gridDim.x * gpw) {
+    const uint64_t grp = g0 + lg;
+    const bool active = in_group && grp < ngroups;
+    const uint64_t t = grp * Ls + s;  // chunk index in memory order
+    const uint32_t kch = (uint32_t)((grp / nrhs) % NCH);  // chunk of the spinor this group holds
+    uint32_t pos[H];
+#pragma unroll
+    for (int h = 0; h < H; h++)  // P+ (reals 0..11) hops down in s, P- (12..23) up; dag exchanges them
+      pos[h] = ((kch * R + h * SV) < 12) != (dag != 0) ? s : Ls - 1 - s;
+    if (active) {
+      A xv[R];
+      dev::load_chunk<P, A>(x, t, xv);
+#pragma unroll
+      for (int h = 0; h < H; h++) {
+        AV e;
+#pragma unroll
+        for (int j = 0; j < SV; j++) e[j] = xv[h * SV + j];
+        AV *col = sx + (lg * H + h) * 2 * Ls + pos[h];
+        col[0] = e;
+        col[Ls] = e;
+      }
+    }
+    __syncthreads();
+    if (active) {
+      A v[R];
+#pragma unroll
+      for (int h = 0; h < H; h++) {
+        const AV *col = sx + (lg * H + h) * 2 * Ls + pos[h] + Ls;
+        A acc[SV];
+#pragma unroll
+        for (int j = 0; j < SV; j++) acc[j] = (A)0;
+        A w = dinv;
+#pragma unroll 4
+        for (uint32_t k = 0; k < Ls; k++) {
+          const A c = k > pos[h] ? -mass * w : w;  // -mass once L^k wraps
+          const AV e = *(col - k);
+#pragma unroll
+          for (int j = 0; j < SV; j++) acc[j] += c * e[j];
+          w *= dinv;
+        }
+#pragma unroll
+        for (int j = 0; j < SV; j++) v[h * SV + j] = alpha * (acc[j] * gnorm);
       }
       if (z) {
         A zv[R];
@@ -121,9 +182,9 @@ void launch_s5(bool inv, const void *x, void *out, const void *z, uint64_t ngrou
   if (nb > (1u << 20)) nb = 1u << 20;
   const dim3 grid((unsigned)nb), block(gpw * Ls);
   if (inv)
-    hipLaunchKernelGGL((k_dwf_s5<P, true>), grid, block, lds, st, x, out, z, ngroups, Ls, nrhs, gpw, d, mass, alpha, beta, dag);
+    hipLaunchKernelGGL((k_dwf_s5_inv<P>), grid, block, 2 * lds, st, x, out, z, ngroups, Ls, nrhs, gpw, d, mass, alpha, beta, dag);
   else
-    hipLaunchKernelGGL((k_dwf_s5<P, false>), grid, block, lds, st, x, out, z, ngroups, Ls, nrhs, gpw, d, mass, alpha, beta,
+    hipLaunchKernelGGL((k_dwf_s5<P>), grid, block, lds, st, x, out, z, ngroups, Ls, nrhs, gpw, d, mass, alpha, beta,
                        dag);
 }
 
