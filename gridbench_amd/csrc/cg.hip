@@ -203,10 +203,7 @@ void launch_xpay(double b, const gbx_spinor_s *r, gbx_spinor_s *p, hipStream_t s
 // with cached output stores, since the solver reads its outputs back at once.
 dhop_cfg solver_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
 {
-  gbx_kcfg k;
-  gbx_dhop_get_cfg((gbx_gauge)u, (gbx_spinor)in, &k);
-  dhop_cfg c = dhop_default_cfg(u, in);
-  if (k.kind == 0) c = dhop_cfg{k.spw, k.threads, k.xcd, 0, k.mc, k.pf, k.wgpc, k.cblk};
+  dhop_cfg c = dhop_fused_cfg(u, in);
   c.nt = 0;
   return c;
 }

@@ -182,39 +182,66 @@ bool dhop_lookup_cfg(const std::string &sig, gbx_kcfg *c)
   return true;
 }
 
+// The shape of a problem nobody tuned: a rule fitted to 300 shapes (extents
+// 4..24, Ls 4..20, 1..16 right-hand sides, whole lattices and red-black
+// halves), each timed in 30 configurations: on fresh shapes it is 2.4 % slower
+// than the best of the 30 on average (25 % at worst); one workgroup of 256 or
+// more threads without the pipeline, whatever the size, was 18 % (89 %).
+//  * mc: above 88 minor indices (16-bit: 128) a workgroup takes chunks of
+//    40..88 of them, whole 128-byte lines, the size that leaves the fewest
+//    lanes idle: a smaller set of neighbours in flight, which the L2s hold
+//    (24 KB a site otherwise).  FP64 16^4 x Ls16 x 8: 1517 us whole, 1110 us
+//    in chunks of 64.
+//  * threads: one wavefront for FP64 and for FP32 fields of up to 2^20
+//    points (more workgroups, no barrier between wavefronts), 256 threads
+//    otherwise, where the links of more sites are staged together; with one
+//    or two sites in a wavefront, a larger workgroup if it idles fewer lanes.
+//  * pf: the gather pipeline pays for its registers (FP64 2 wavefronts a SIMD
+//    instead of 4, FP32 5 instead of 8) except where the whole grid is resident
+//    in one round without it and not with it, and with 16-bit storage once
+//    the grid fills the card.
 dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
 {
-  (void)u;
-  dhop_cfg c;
+  const bool f64 = in->prec == GBX_F64, f32 = in->prec == GBX_F32, f16 = !f64 && !f32;
   const uint32_t M = in->M;
-  // LDS per workgroup stays <= 40 KB so several workgroups share a CU.
-  const int spw_max = in->prec == GBX_F64 ? 32 : 64;
-  // Prefer a workgroup of exactly spw*M threads, a multiple of 64, near 256.
-  int spw = 0;
-  for (int s = 1; s <= spw_max; s++) {
-    const uint32_t t = (uint32_t)s * M;
-    if (t > 1024) break;
-    if (t % 64 == 0 && t >= 256) {
-      spw = s;
-      break;
-    }
-  }
-  if (spw) {
-    c.spw = spw;
-    c.threads = (int)(spw * M);
-  } else if (M >= 256) {
-    c.spw = 1;
-    c.threads = 256;
+  const uint64_t vol = u->geom->vol, pts = vol * (uint64_t)M;
+  // Sites of a t-thread workgroup at chunk m: the LDS for their links leaves
+  // room for the wavefronts the registers allow.
+  auto sites = [&](uint32_t t, uint32_t m) { return std::min(t / m, f64 ? t / 4 : t * 3 / 16); };
+  uint32_t mc = M, spw = 1, threads = 256;
+  if (M > (f16 ? 128u : 88u)) {
+    uint64_t best = ~0ull;
+    for (uint32_t m : {64, 56, 72, 48, 80, 40, 88})
+      for (uint32_t t = 256; t >= 64; t -= 64) {
+        const uint32_t n = sites(t, m);
+        // lanes per site, in units that keep the division exact enough
+        const uint64_t lanes = n ? (uint64_t)((M + m - 1) / m) * t * 4096 / n : ~0ull;
+        if (lanes < best) {
+          best = lanes;
+          mc = m;
+          spw = n;
+          threads = t;
+        }
+      }
+  } else if (M > 64) {
+    threads = f16 && M <= 85 ? 256 : 128;
+    spw = sites(threads, M);
   } else {
-    c.spw = (int)((256 + M - 1) / M);
-    if (c.spw > spw_max) c.spw = spw_max;
-    c.threads = (int)(((uint32_t)c.spw * M + 63) / 64 * 64);
-    if (c.threads > 1024) c.threads = 1024;
+    threads = f64 || (f32 && M >= 8 && pts <= (1u << 20)) || (f32 && pts <= 50000) ? 64 : 256;
+    while (threads < 256 && sites(threads, M) * M * 5 < threads * 3) threads += 64;  // 3/5 of the lanes busy
+    spw = sites(threads, M);
   }
+  const uint64_t waves = (vol + spw - 1) / spw * ((M + mc - 1) / mc) * (threads / 64);
+  dhop_cfg c;
+  c.spw = (int)spw;
+  c.threads = (int)threads;
   c.xcd = 1;
   c.nt = 1;
-  c.mc = 0;
-  c.pf = 0;
+  c.mc = mc == M ? 0 : (int)mc;
+  if (f64) c.pf = waves > 2048 && waves <= (M < 16 ? 3584u : 3072u) ? 0 : M <= 24 ? 1 : 2;
+  else if (f32) c.pf = M <= 16 && waves > 5120 && waves <= 8192 ? 0 : M <= 24 ? 1 : 2;
+  else c.pf = waves <= 2048 ? 2 : 0;
+  c.axpby_pf = true;
   c.wgpc = 0;
   c.cblk = 0;
   return c;
@@ -385,9 +412,19 @@ static dhop_cfg exact_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
   if (M <= target) {
     c.spw = (int)(target / M);
     c.threads = (int)(((uint32_t)c.spw * M + 63) / 64 * 64);
+    c.mc = 0;
     c.pf = 1;
   }
   return c;
+}
+
+// The VALU kernel's shape for the fused forms: the tuned one if a VALU shape
+// was tuned (without its gather pipeline, which was timed on the plain form),
+// else the default.
+dhop_cfg dhop_fused_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
+{
+  gbx_kcfg k;
+  return dhop_lookup_cfg(dhop_signature(u, in), &k) && k.kind == 0 ? from_kcfg(k) : dhop_default_cfg(u, in);
 }
 
 int dhop_run_exact(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in, int dag, hipStream_t st)
@@ -484,10 +521,7 @@ extern "C" int gbx_dhop_xpay(gbx_gauge u, gbx_spinor out, gbx_spinor x, gbx_spin
   GBX_TRY(check_operands(u, out, in));
   GBX_CHECK(x, GBX_ENULL, "gbx_dhop_xpay: NULL field x");
   GBX_CHECK(dag == 0 || dag == 1, GBX_EINVAL, "gbx_dhop_xpay: dag must be 0 or 1");
-  gbx_kcfg k;
-  gbx_dhop_get_cfg(u, in, &k);
-  if (k.kind != 0) k = to_kcfg(dhop_default_cfg(u, in));
-  return dhop_launch(u, out, in, dag, from_kcfg(k), alpha, beta, x, u->geom->stream);
+  return dhop_launch(u, out, in, dag, dhop_fused_cfg(u, in), alpha, beta, x, u->geom->stream);
 }
 
 extern "C" int gbx_dhop_xpay_cfg(gbx_gauge u, gbx_spinor out, gbx_spinor x, gbx_spinor in, int dag, double alpha,

@@ -180,9 +180,9 @@ struct dhop_cfg {
   int pf;        // 1: two-buffer gather pipeline (workgroups of <= 256 threads)
   int wgpc;      // cap on resident workgroups per CU via padded LDS (0 = none)
   int cblk;      // site groups per minor-chunk cycle (0 = whole lattice per chunk)
-  // The fused axpby form runs without the gather pipeline (its tuned pf is
-  // that of the plain kernel, and the extra centre loads make the pipeline
-  // slower there) unless the caller asked for a pf explicitly.
+  // The fused axpby form runs without a tuned shape's gather pipeline (its pf
+  // was timed on the plain kernel, without the centre loads) unless the caller
+  // asked for a pf explicitly or the shape is the default one.
   bool axpby_pf = false;
   // The field's ghosts hold spin-projected halves (a domain part's face
   // slots after gbx_halo_ghost_proj receives).
@@ -205,6 +205,7 @@ int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in,
 // Dhop with the reference's rounding, on the problem's tuned VALU shape.
 int dhop_run_exact(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in, int dag, hipStream_t st);
 dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in);
+dhop_cfg dhop_fused_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in);
 int dhop_cfg_check(const dhop_cfg &cfg, const gbx_gauge_s *u, const gbx_spinor_s *in);
 // LDS-tiled kernel (kind 2): out = Dhop(in) on a whole lattice.
 int tile_cfg_check(const gbx_kcfg &k, const gbx_gauge_s *u, const gbx_spinor_s *in);
