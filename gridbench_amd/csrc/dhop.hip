@@ -15,84 +15,20 @@
 #include <mutex>
 #include <unordered_map>
 
-#include "dhop_dev.h"
-#include "gbx_internal.h"
+#include "dhop_kernel.h"
 
 namespace {
 
-// Logical workgroup L covers sites q0 .. q0+spw-1 (site block L % nwg_sites)
-// and minor indices m0 .. m0+mc-1 (minor chunk L / nwg_sites): with mc < M
-// the lattice is swept once per minor chunk, so the 8-neighbour working set
-// is that of an mc-wide field (the links are re-read once per chunk).
-// GP: a domain part whose ghosts hold spin-projected halves from ghost0 on
-// (dhop_site_gp).  TD: fields in the GBX_BASIS_TDIAG spin basis.
-template <int P, bool DAG, bool C12, bool AXPBY, int PF, bool EXACT = false, bool GP = false, bool TD = false>
-__global__ void __launch_bounds__(PF ? 256 : 1024)
-    k_dhop(const void *__restrict__ gauge, const uint32_t *__restrict__ nbr, const void *__restrict__ in,
-           void *__restrict__ out, const void *__restrict__ center, uint32_t nslot, uint32_t M, uint32_t spw, uint32_t mc,
-           uint32_t nwg_sites, uint32_t cblk, uint32_t nchunk, uint32_t nwg, uint32_t per_xcd, int xcd, int nt,
-           typename dev::Traits<P>::acc alpha,
-           typename dev::Traits<P>::acc beta, uint32_t ghost0)
-{
-  typedef typename dev::Traits<P>::acc A;
-  extern __shared__ __align__(16) unsigned char smem[];
-  A *sU = (A *)smem;
-  uint32_t *sN = (uint32_t *)(sU + (size_t)spw * 8 * 18);
-
-  const uint32_t L = xcd ? (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
-  if (L >= nwg) return;  // uniform over the workgroup, before any barrier
-  // cblk site groups are visited for every minor chunk before the next
-  // cblk groups (chunk-inner order); cblk == nwg_sites sweeps the lattice
-  // once per chunk (chunk-outer order).
-  const uint32_t per = cblk * nchunk, grp = L / per, r = L - grp * per;
-  const uint32_t chunk = r / cblk, b = grp * cblk + (r - chunk * cblk);
-  if (b >= nwg_sites) return;
-  const uint32_t q0 = b * spw, m0 = chunk * mc;
-  const uint32_t nsl = min(spw, nslot - q0), mcc = min(mc, M - m0);
-  dev::stage_links<P, C12>(gauge, nbr, q0, nsl, sU, sN);
-
-  const uint32_t items = nsl * mcc;
-  for (uint32_t w = threadIdx.x; w < items; w += blockDim.x) {
-    const uint32_t sl = w / mcc, m = m0 + (w - sl * mcc);
-    A rr[12], ri[12];
-    if constexpr (GP) dev::dhop_site_gp<P, DAG, PF>(in, sN + sl * 8, M, m, ghost0, sU + sl * 8 * 18, rr, ri);
-    else dev::dhop_site<P, DAG, PF, EXACT, TD>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
-    dev::store_site<P, AXPBY>(out, center, q0 + sl, M, m, rr, ri, alpha, beta, nt != 0);
-  }
-}
-
-struct LaunchArgs {
-  dim3 grid, block;
-  size_t lds;
-  hipStream_t st;
-  const void *gauge;
-  const uint32_t *nbr;
-  const void *in;
-  void *out;
-  const void *center;
-  uint32_t nslot, M, spw, mc, nwg_sites, cblk, nchunk, nwg, per_xcd;
-  int xcd, nt;
-  double alpha, beta;
-  uint32_t ghost0;
-};
-
-template <int P, bool DAG, bool C12, bool AXPBY, int PF, bool EXACT = false, bool GP = false, bool TD = false>
-void launch_t(const LaunchArgs &a)
-{
-  typedef typename dev::Traits<P>::acc A;
-  hipLaunchKernelGGL((k_dhop<P, DAG, C12, AXPBY, PF, EXACT, GP, TD>), a.grid, a.block, a.lds, a.st, a.gauge, a.nbr, a.in, a.out,
-                     a.center, a.nslot, a.M, a.spw, a.mc, a.nwg_sites, a.cblk, a.nchunk, a.nwg, a.per_xcd, a.xcd, a.nt,
-                     (A)a.alpha, (A)a.beta, a.ghost0);
-}
+using namespace dhopk;
 
 // Projected ghosts (FP64 / FP32, no axpby).
 template <int P>
 void launch_gp(bool dag, bool c12, int pf, const LaunchArgs &a)
 {
 #define GBX_GP(D_, C_)                                        \
-  if (pf == 2) launch_t<P, D_, C_, false, 2, false, true>(a); \
-  else if (pf == 1) launch_t<P, D_, C_, false, 1, false, true>(a); \
-  else launch_t<P, D_, C_, false, 0, false, true>(a);
+  if (pf == 2) launch_t<P, D_, C_, EPI_STORE, 2, false, true>(a); \
+  else if (pf == 1) launch_t<P, D_, C_, EPI_STORE, 1, false, true>(a); \
+  else launch_t<P, D_, C_, EPI_STORE, 0, false, true>(a);
   if (dag) {
     if (c12) { GBX_GP(true, true) } else { GBX_GP(true, false) }
   } else {
@@ -105,12 +41,12 @@ template <int P, bool DAG, bool C12, bool TD = false>
 void launch_dc(bool axpby, int pf, const LaunchArgs &a)
 {
   if (axpby) {
-    if (pf == 2) launch_t<P, DAG, C12, true, 2, false, false, TD>(a);
-    else if (pf == 1) launch_t<P, DAG, C12, true, 1, false, false, TD>(a);
-    else launch_t<P, DAG, C12, true, 0, false, false, TD>(a);
-  } else if (pf == 2) launch_t<P, DAG, C12, false, 2, false, false, TD>(a);
-  else if (pf == 1) launch_t<P, DAG, C12, false, 1, false, false, TD>(a);
-  else launch_t<P, DAG, C12, false, 0, false, false, TD>(a);
+    if (pf == 2) launch_t<P, DAG, C12, EPI_AXPBY, 2, false, false, TD>(a);
+    else if (pf == 1) launch_t<P, DAG, C12, EPI_AXPBY, 1, false, false, TD>(a);
+    else launch_t<P, DAG, C12, EPI_AXPBY, 0, false, false, TD>(a);
+  } else if (pf == 2) launch_t<P, DAG, C12, EPI_STORE, 2, false, false, TD>(a);
+  else if (pf == 1) launch_t<P, DAG, C12, EPI_STORE, 1, false, false, TD>(a);
+  else launch_t<P, DAG, C12, EPI_STORE, 0, false, false, TD>(a);
 }
 
 template <int P, bool TD = false>
@@ -127,13 +63,13 @@ template <int P>
 void launch_exact(bool dag, int pf, const LaunchArgs &a)
 {
   if (dag) {
-    if (pf == 2) launch_t<P, true, false, false, 2, true>(a);
-    else if (pf == 1) launch_t<P, true, false, false, 1, true>(a);
-    else launch_t<P, true, false, false, 0, true>(a);
+    if (pf == 2) launch_t<P, true, false, EPI_STORE, 2, true>(a);
+    else if (pf == 1) launch_t<P, true, false, EPI_STORE, 1, true>(a);
+    else launch_t<P, true, false, EPI_STORE, 0, true>(a);
   } else {
-    if (pf == 2) launch_t<P, false, false, false, 2, true>(a);
-    else if (pf == 1) launch_t<P, false, false, false, 1, true>(a);
-    else launch_t<P, false, false, false, 0, true>(a);
+    if (pf == 2) launch_t<P, false, false, EPI_STORE, 2, true>(a);
+    else if (pf == 1) launch_t<P, false, false, EPI_STORE, 1, true>(a);
+    else launch_t<P, false, false, EPI_STORE, 0, true>(a);
   }
 }
 
@@ -261,6 +197,19 @@ int dhop_cfg_check(const dhop_cfg &c, const gbx_gauge_s *u, const gbx_spinor_s *
   return GBX_OK;
 }
 
+bool dhop_s5inv_fits(const gbx_spinor_s *in, const dhop_cfg &c)
+{
+  return (c.mc <= 0 || (uint32_t)c.mc >= in->M) && (uint64_t)c.spw * in->M <= (uint64_t)c.threads;
+}
+
+uint32_t dhop_workgroups(const gbx_gauge_s *u, const gbx_spinor_s *in, const dhop_cfg &c)
+{
+  const uint32_t spw = (uint32_t)c.spw, mc = (c.mc <= 0 || (uint32_t)c.mc > in->M) ? in->M : (uint32_t)c.mc;
+  const uint32_t sites = (uint32_t)((u->geom->vol + spw - 1) / spw), chunks = (in->M + mc - 1) / mc;
+  const uint32_t cblk = (c.cblk <= 0 || (uint32_t)c.cblk >= sites) ? sites : (uint32_t)c.cblk;
+  return (sites + cblk - 1) / cblk * cblk * chunks;
+}
+
 static int check_operands(const gbx_gauge_s *u, const gbx_spinor_s *out, const gbx_spinor_s *in)
 {
   GBX_CHECK(u && out && in, GBX_ENULL, "dhop: NULL handle");
@@ -277,11 +226,13 @@ static int check_operands(const gbx_gauge_s *u, const gbx_spinor_s *out, const g
 }
 
 int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in, int dag, const dhop_cfg &c, double alpha,
-                double beta, const gbx_spinor_s *center, hipStream_t st, bool exact, SlotRange range)
+                double beta, const gbx_spinor_s *center, hipStream_t st, bool exact, SlotRange range, const dhop_fuse *fuse)
 {
   GBX_TRY(check_operands(u, out, in));
   GBX_TRY(dhop_cfg_check(c, u, in));
-  const bool axpby = !(alpha == 0.0 && beta == 1.0);
+  const int s5 = fuse ? fuse->s5 : (int)dhop_fuse::NONE;
+  const bool axpby = s5 == dhop_fuse::MOOEE || (s5 == dhop_fuse::NONE && !(alpha == 0.0 && beta == 1.0));
+  const bool red = fuse && fuse->partial;
   GBX_CHECK(!exact || ((u->prec == GBX_F64 || u->prec == GBX_F32) && !u->comp12 && !axpby), GBX_EUNSUPPORTED,
             "dhop: the reference-rounding kernel takes FP64 / FP32 fields with 18-real links");
   const bool td = in->basis == GBX_BASIS_TDIAG;
@@ -336,6 +287,29 @@ int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in,
   a.beta = beta;
   a.ghost0 = (uint32_t)u->geom->vol;
   const int pf = (axpby && !c.axpby_pf) ? 0 : c.pf;
+  if (fuse) {
+    a.skip = fuse->skip;
+    a.partial = fuse->partial;
+  }
+  if (s5 != dhop_fuse::NONE || red) {
+    GBX_CHECK(whole && !exact && !c.projected_ghosts && (!red || (axpby && !dag)) && (s5 == dhop_fuse::NONE || !td),
+              GBX_EUNSUPPORTED, "dhop: no such fused form");
+    int epi = EPI_AXPBY;
+    if (s5 != dhop_fuse::NONE) {
+      a.d = 5.0 - fuse->dwf->M5;
+      a.mass = fuse->dwf->mass;
+      a.Ls = (uint32_t)in->Ls;
+      epi = EPI_S5;
+    }
+    if (s5 == dhop_fuse::MOOEE_INV) {
+      GBX_CHECK(dhop_s5inv_fits(in, c), GBX_EUNSUPPORTED, "dhop: Mooee^-1 does not fit this launch shape");
+      a.lds = std::max(a.lds, (size_t)c.threads * 12 * (u->prec == GBX_F64 ? 8 : 4));
+      epi = EPI_S5INV;
+    }
+    launch_fused(u->prec, epi, dag != 0, u->comp12 != 0, td, red, pf, a);
+    GBX_HIP(hipGetLastError());
+    return GBX_OK;
+  }
   if (c.projected_ghosts) {
     GBX_CHECK((u->prec == GBX_F64 || u->prec == GBX_F32) && !axpby && !exact && u->geom->nghost, GBX_EUNSUPPORTED,
               "dhop: projected ghosts need a domain part, FP64 / FP32 fields and no axpby");

@@ -483,10 +483,11 @@ __device__ __forceinline__ void dhop_site_gp(const void *__restrict__ in, const 
   }
 }
 
-// Write the 4-spinor result (optionally out = alpha*center + beta*result).
+// Write the 4-spinor result (optionally out = alpha*center + beta*result,
+// which then replaces the result in rr, ri).
 template <int P, bool AXPBY>
 __device__ __forceinline__ void store_site(void *__restrict__ out, const void *__restrict__ center, uint32_t q, uint32_t M,
-                                           uint32_t m, const typename Traits<P>::acc *rr, const typename Traits<P>::acc *ri,
+                                           uint32_t m, typename Traits<P>::acc *rr, typename Traits<P>::acc *ri,
                                            typename Traits<P>::acc alpha, typename Traits<P>::acc beta, bool nt)
 {
   typedef typename Traits<P>::acc A;
@@ -504,7 +505,12 @@ __device__ __forceinline__ void store_site(void *__restrict__ out, const void *_
       A c[R];
       load_chunk<P, A>(center, base + (uint64_t)k * M, c);
 #pragma unroll
-      for (int j = 0; j < R; j++) v[j] = alpha * c[j] + beta * v[j];
+      for (int j = 0; j < R; j++) {
+        const int r = k * R + j;
+        v[j] = alpha * c[j] + beta * v[j];
+        if (r & 1) ri[r >> 1] = v[j];
+        else rr[r >> 1] = v[j];
+      }
     }
     store_chunk<P, A>(out, base + (uint64_t)k * M, v, nt);
   }

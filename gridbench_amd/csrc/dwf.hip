@@ -18,7 +18,7 @@
 // mass 0.1 and M5 1.0 (TableGenerate.cc:47-50) and writes out only its Dhop;
 // the terms here are the Shamir form of that operator.
 //
-// Kernel: one thread per 16-byte chunk of the SoA layout.  Chunks are stored
+// Kernels: one thread per 16-byte chunk of the SoA layout.  Chunks are stored
 // ((q*nch + k)*M + m) with m = rhs*Ls + s, so every Ls consecutive chunks are
 // one (site, chunk, right-hand side) group holding all s-slices.  A
 // workgroup loads whole groups into LDS (coalesced), then each thread forms
@@ -239,15 +239,18 @@ extern "C" int gbx_dwf_mooee(gbx_spinor out, gbx_spinor in, const gbx_dwf_params
   return dwf_s5_launch(out, in, nullptr, p, inv, dag, 1.0, 0.0, in->geom->stream);
 }
 
-// out = D in = Mooee in - (1/2) Dhop in on a whole lattice: out = Dhop in,
-// then out = Mooee in - (1/2) out (the 5th-dimension kernel reads its own
-// output element of z before writing it).
+// out = D in = Mooee in - (1/2) Dhop in on a whole lattice, in one pass: the
+// hopping kernel adds Mooee of its own site's slices to each point it writes.
 extern "C" int gbx_dwf_apply(gbx_gauge u, gbx_spinor out, gbx_spinor in, const gbx_dwf_params *p, int dag)
 {
   GBX_CHECK(u && out && in, GBX_ENULL, "gbx_dwf_apply: NULL argument");
   GBX_CHECK(whole_lattice(u->geom), GBX_EINVAL, "gbx_dwf_apply: whole lattices only (red-black halves: gbx_dwf_solve_eo)");
   GBX_TRY(check_params(p, in->Ls));
   GBX_TRY(require_chiral("gbx_dwf_apply", in));
-  GBX_TRY(gbx_dhop(u, out, in, dag));
-  return dwf_s5_launch(out, in, out, p, 0, dag, 1.0, -0.5, u->geom->stream);
+  GBX_TRY(dhop_check_operands(u, out, in));
+  GBX_CHECK(dag == 0 || dag == 1, GBX_EINVAL, "gbx_dwf_apply: dag must be 0 or 1");
+  dhop_fuse f;
+  f.s5 = dhop_fuse::MOOEE;
+  f.dwf = p;
+  return dhop_launch(u, out, in, dag, dhop_fused_cfg(u, in), 1.0, -0.5, in, u->geom->stream, false, SlotRange(), &f);
 }

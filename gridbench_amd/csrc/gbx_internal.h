@@ -196,12 +196,29 @@ struct SlotRange {
   uint64_t begin = 0, end = UINT64_MAX;
 };
 
+// More of an operator in the hopping kernel's epilogue (VALU kernel, chiral
+// fields for the domain-wall terms).
+struct dhop_fuse {
+  enum { NONE = 0, MOOEE = 1, MOOEE_INV = 2 };
+  // MOOEE: out = Mooee center + beta Dhop(in) (alpha is not used); MOOEE_INV:
+  // out = Mooee^-1 Dhop(in); their adjoints for dag.
+  int s5 = NONE;
+  const gbx_dwf_params *dwf = nullptr;
+  const uint32_t *skip = nullptr;  // device flag: nothing runs once it is not zero
+  // |out|^2 of each workgroup (dag 0, with axpby or MOOEE): dhop_workgroups
+  // values.
+  double *partial = nullptr;
+};
+uint32_t dhop_workgroups(const gbx_gauge_s *u, const gbx_spinor_s *in, const dhop_cfg &cfg);
+// Whether MOOEE_INV can run at this shape: one point per thread, whole columns.
+bool dhop_s5inv_fits(const gbx_spinor_s *in, const dhop_cfg &cfg);
+
 // out = alpha*in_c + beta*Dhop(in) where in_c is `center` (may be null when alpha == 0).
 // exact: the reference's rounding (no fused multiply-adds; FP64 / FP32 fields
 // with 18-real links, no axpby).
 int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in, int dag,
                 const dhop_cfg &cfg, double alpha, double beta, const gbx_spinor_s *center,
-                hipStream_t stream, bool exact = false, SlotRange range = SlotRange());
+                hipStream_t stream, bool exact = false, SlotRange range = SlotRange(), const dhop_fuse *fuse = nullptr);
 // Dhop with the reference's rounding, on the problem's tuned VALU shape.
 int dhop_run_exact(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in, int dag, hipStream_t st);
 dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in);
