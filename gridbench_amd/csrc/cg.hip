@@ -221,21 +221,45 @@ struct NormalOp {
   gbx_spinor_s *t, *to;
   int kind = OP_WILSON;       // red-black only: M = 1 - kappa Dhop, or the DWF operator
   gbx_dwf_params dwf{0, 0};
-  gbx_spinor_s *te = nullptr;  // DWF: a second even-half temporary
 };
+
+// out = Mooee^-1 Dhop in (dag: the adjoints), in one kernel where the launch
+// shape holds whole columns of slices.
+int mooee_inv_dhop(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in, const gbx_dwf_params *dwf, int dag,
+                   hipStream_t st)
+{
+  const dhop_cfg c = solver_cfg(u, in);
+  dhop_fuse f;
+  if (dhop_s5inv_fits(in, c)) {
+    f.s5 = dhop_fuse::MOOEE_INV;
+    f.dwf = dwf;
+    return dhop_launch(u, out, in, dag, c, 0.0, 1.0, nullptr, st, false, SlotRange(), &f);
+  }
+  GBX_TRY(dhop_launch(u, out, in, dag, c, 0.0, 1.0, nullptr, st));
+  return dwf_s5_launch(out, out, nullptr, dwf, 1, dag, 1.0, 0.0, st);
+}
+
+// out = Mooee c + beta Dhop in (dag: the adjoints) in one kernel.
+int mooee_plus_dhop(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *c, const gbx_spinor_s *in,
+                    const gbx_dwf_params *dwf, int dag, double beta, hipStream_t st)
+{
+  dhop_fuse f;
+  f.s5 = dhop_fuse::MOOEE;
+  f.dwf = dwf;
+  return dhop_launch(u, out, in, dag, solver_cfg(u, in), 1.0, beta, c, st, false, SlotRange(), &f);
+}
 
 // y = Mpc x (dag = 0) or Mpc^dag x (dag = 1), with dagger kernels for dag
 // ((DhopEO DhopOE)^dag = (Dhop^dag)_EO (Dhop^dag)_OE):
 //   Wilson:  to = DhopOE x;  y = x - kappa^2 DhopEO to
-//   DWF:     to = Mooee^-1 DhopOE x;  te = DhopEO to;  y = Mooee x - te / 4
+//   DWF:     to = Mooee^-1 DhopOE x;  y = Mooee x - DhopEO to / 4
 int apply_schur(const NormalOp &op, gbx_spinor_s *y, const gbx_spinor_s *x, int dag, hipStream_t st)
 {
-  GBX_TRY(dhop_launch(op.uo, op.to, x, dag, solver_cfg(op.uo, x), 0.0, 1.0, nullptr, st));
   if (op.kind == OP_DWF) {
-    GBX_TRY(dwf_s5_launch(op.to, op.to, nullptr, &op.dwf, 1, dag, 1.0, 0.0, st));
-    GBX_TRY(dhop_launch(op.ue, op.te, op.to, dag, solver_cfg(op.ue, op.to), 0.0, 1.0, nullptr, st));
-    return dwf_s5_launch(y, x, op.te, &op.dwf, 0, dag, 1.0, -0.25, st);
+    GBX_TRY(mooee_inv_dhop(op.uo, op.to, x, &op.dwf, dag, st));
+    return mooee_plus_dhop(op.ue, y, x, op.to, &op.dwf, dag, -0.25, st);
   }
+  GBX_TRY(dhop_launch(op.uo, op.to, x, dag, solver_cfg(op.uo, x), 0.0, 1.0, nullptr, st));
   GBX_TRY(dhop_launch(op.ue, y, op.to, dag, solver_cfg(op.ue, op.to), 1.0, -op.kappa * op.kappa, x, st));
   return GBX_OK;
 }
@@ -461,14 +485,13 @@ int solve_schur(int kind, const gbx_dwf_params *dwf, const gbx_gauge_s *const u_
   const double kappa = prm->kappa;
   const int plo = u_lo ? u_lo[0]->prec : GBX_F64;
   const int pe = u_lo ? GBX_F32 : GBX_F64;
-  Tmp bp, r, y, t, te, to, e, ri, p, Ap, tl, tel, tol_, ro;
+  Tmp bp, r, y, t, to, e, ri, p, Ap, tl, tol_, ro;
   Scratch sc;
   GBX_TRY(sc.init());
   GBX_TRY(make(g, Ls, GBX_F64, bp));
   GBX_TRY(make(g, Ls, GBX_F64, r));
   GBX_TRY(make(g, Ls, GBX_F64, y));
   GBX_TRY(make(g, Ls, GBX_F64, t));
-  GBX_TRY(make(g, Ls, GBX_F64, te));
   GBX_TRY(make(g1, Ls, GBX_F64, to));
   GBX_TRY(make(g1, Ls, GBX_F64, ro));
   GBX_TRY(make(g, Ls, pe, e));
@@ -476,17 +499,14 @@ int solve_schur(int kind, const gbx_dwf_params *dwf, const gbx_gauge_s *const u_
   GBX_TRY(make(g, Ls, plo, p));
   GBX_TRY(make(g, Ls, plo, Ap));
   GBX_TRY(make(g, Ls, plo, tl));
-  GBX_TRY(make(g, Ls, plo, tel));
   GBX_TRY(make(g1, Ls, plo, tol_));
-  for (Tmp *f : {&bp, &r, &y, &t, &te, &to, &ro, &e, &ri, &p, &Ap, &tl, &tel, &tol_}) f->s->basis = basis;
+  for (Tmp *f : {&bp, &r, &y, &t, &to, &ro, &e, &ri, &p, &Ap, &tl, &tol_}) f->s->basis = basis;
   NormalOp op_hi{true, u_hi[0], u_hi[1], kappa, t.s, to.s};
   NormalOp op_lo = u_lo ? NormalOp{true, u_lo[0], u_lo[1], kappa, tl.s, tol_.s} : NormalOp{true, u_hi[0], u_hi[1], kappa, tl.s,
                                                                                            tol_.s};
   op_hi.kind = op_lo.kind = kind;
   if (kind == OP_DWF) {
     op_hi.dwf = op_lo.dwf = *dwf;
-    op_hi.te = te.s;
-    op_lo.te = tel.s;
   }
   double bbe, bbo;
   GBX_TRY(spinor_norm2_on(b[0], &bbe, s));
@@ -527,10 +547,8 @@ int solve_schur(int kind, const gbx_dwf_params *dwf, const gbx_gauge_s *const u_
     // x_o = Mooee^-1 (b_o + DhopOE x_e / 2); then b - D x with D = Mooee - Dhop / 2
     GBX_TRY(xpay(u_hi[1], to.s, b[1], x[0], 0, 1.0, 0.5, s));
     GBX_TRY(dwf_s5_launch(x[1], to.s, nullptr, dwf, 1, 0, 1.0, 0.0, s));
-    GBX_TRY(dhop_launch(u_hi[0], te.s, x[1], 0, solver_cfg(u_hi[0], x[1]), 0.0, 1.0, nullptr, s));
-    GBX_TRY(dwf_s5_launch(y.s, x[0], te.s, dwf, 0, 0, 1.0, -0.5, s));  // (D x)_e
-    GBX_TRY(dhop_launch(u_hi[1], to.s, x[0], 0, solver_cfg(u_hi[1], x[0]), 0.0, 1.0, nullptr, s));
-    GBX_TRY(dwf_s5_launch(to.s, x[1], to.s, dwf, 0, 0, 1.0, -0.5, s));  // (D x)_o
+    GBX_TRY(mooee_plus_dhop(u_hi[0], y.s, x[0], x[1], dwf, 0, -0.5, s));   // (D x)_e
+    GBX_TRY(mooee_plus_dhop(u_hi[1], to.s, x[1], x[0], dwf, 0, -0.5, s));  // (D x)_o
   } else {
     // x_o = b_o + kappa DhopOE x_e; then b - M x
     GBX_TRY(xpay(u_hi[1], x[1], b[1], x[0], 0, 1.0, kappa, s));

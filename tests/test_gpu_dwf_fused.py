@@ -44,3 +44,22 @@ def test_operator_with_compressed_links(gpu, gbx):
         gbx.dwf_apply(U, y, x)
         out.append(y.download())
     assert rel_l2(out[1], out[0]) <= 1e-14
+
+
+@pytest.mark.parametrize("Ls", [2, 5, 17, 64, 96])  # 96: sliced in minor chunks, Mooee^-1 in a kernel of its own
+@pytest.mark.parametrize("lo", [None, "f32", "f16"])
+def test_even_odd_solve_at_the_edges_of_its_shapes(gpu, gbx, Ls, lo):
+    dims = (4, 2, 4, 2)
+    dbl, psi = gbx.gen_doubled_gauge(dims, 95), gbx.gen_spinor(dims, Ls, 1, 96)
+    pair = gbx.Geometry.rb_pair(dims)
+    U = [gbx.GaugeField(g, "f64").upload(dbl) for g in pair]
+    low = None if lo is None else [gbx.GaugeField(g, lo).upload(dbl) for g in pair]
+    b = [gbx.SpinorField(g, Ls, 1, "f64").upload(h) for g, h in zip(pair, gbx.rb_split(dims, psi))]
+    x = [gbx.SpinorField(g, Ls, 1, "f64").zero() for g in pair]
+    st = gbx.dwf_solve_eo(U, low, x, b, tol=1e-10, max_outer=60)
+    assert st["true_resid"] <= 1e-10
+    g = gbx.Geometry(dims)
+    xl = gbx.SpinorField(g, Ls, 1, "f64").upload(gbx.rb_merge(dims, x[0].download(), x[1].download()))
+    y = gbx.dhop(gbx.GaugeField(g, "f64").upload(dbl), gbx.SpinorField(g, Ls, 1, "f64"), xl)
+    Dx = mooee_np(xl.download(), M5, MASS) - 0.5 * y.download()
+    assert rel_l2(Dx, psi) <= 2e-10
