@@ -289,9 +289,11 @@ int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in,
   const int pf = (axpby && !c.axpby_pf) ? 0 : c.pf;
   if (fuse) {
     a.skip = fuse->skip;
+    a.skip_at = fuse->skip_at;
     a.partial = fuse->partial;
   }
   if (s5 != dhop_fuse::NONE || red) {
+    a.lds = std::min(a.lds, (size_t)160 * 1024 - 128);  // a residency pad leaves room for the sum's scratch
     GBX_CHECK(whole && !exact && !c.projected_ghosts && (!red || (axpby && !dag)) && (s5 == dhop_fuse::NONE || !td),
               GBX_EUNSUPPORTED, "dhop: no such fused form");
     int epi = EPI_AXPBY;

@@ -21,7 +21,8 @@ template <typename A> struct Epi {
   A alpha, beta;
   A d, mass;             // domain-wall terms: d = 5 - M5
   uint32_t Ls;
-  const uint32_t *skip;  // nothing runs if *skip is not zero
+  const uint32_t *skip;  // nothing runs if *skip <= skip_at
+  uint32_t skip_at;
   double *partial;       // RED: |out|^2 of every workgroup
 };
 
@@ -158,7 +159,7 @@ __global__ void __launch_bounds__(PF ? 256 : 1024)
 
   const uint32_t L = xcd ? (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
   if (L >= nwg) return;  // uniform over the workgroup, before any barrier
-  if (e.skip && *e.skip) return;
+  if (e.skip && *e.skip <= e.skip_at) return;
   // cblk site groups are visited for every minor chunk before the next
   // cblk groups (chunk-inner order); cblk == nwg_sites sweeps the lattice
   // once per chunk (chunk-outer order).
@@ -219,6 +220,7 @@ struct LaunchArgs {
   double d = 0, mass = 0;
   uint32_t Ls = 1;
   const uint32_t *skip = nullptr;
+  uint32_t skip_at = 0;
   double *partial = nullptr;
 };
 
@@ -226,7 +228,7 @@ template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT = false, bool G
 void launch_t(const LaunchArgs &a)
 {
   typedef typename dev::Traits<P>::acc A;
-  const Epi<A> e{(A)a.alpha, (A)a.beta, (A)a.d, (A)a.mass, a.Ls, a.skip, a.partial};
+  const Epi<A> e{(A)a.alpha, (A)a.beta, (A)a.d, (A)a.mass, a.Ls, a.skip, a.skip_at, a.partial};
   hipLaunchKernelGGL((k_dhop<P, DAG, C12, EPI, PF, EXACT, GP, TD, RED>), a.grid, a.block, a.lds, a.st, a.gauge, a.nbr, a.in,
                      a.out, a.center, a.nslot, a.M, a.spw, a.mc, a.nwg_sites, a.cblk, a.nchunk, a.nwg, a.per_xcd, a.xcd, a.nt,
                      e, a.ghost0);

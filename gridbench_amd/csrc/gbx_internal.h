@@ -204,7 +204,8 @@ struct dhop_fuse {
   // out = Mooee^-1 Dhop(in); their adjoints for dag.
   int s5 = NONE;
   const gbx_dwf_params *dwf = nullptr;
-  const uint32_t *skip = nullptr;  // device flag: nothing runs once it is not zero
+  const uint32_t *skip = nullptr;  // device word: nothing runs if *skip <= skip_at
+  uint32_t skip_at = 0;
   // |out|^2 of each workgroup (dag 0, with axpby or MOOEE): dhop_workgroups
   // values.
   double *partial = nullptr;
