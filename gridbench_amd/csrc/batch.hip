@@ -216,13 +216,27 @@ namespace {
 
 size_t lds_for(int prec, uint32_t spw) { return (size_t)spw * 8 * 18 * (prec == GBX_F64 ? 8 : 4) + (size_t)spw * 8 * 4; }
 
-// Sites per work item for a lattice of minor extent M: about `points`
-// (site, minor) points, at most 64 sites.
+// Sites per work item for a lattice of minor extent M: at most `points`
+// (site, minor) points (one site if it has more), at most 64 sites.  Rounded
+// down: a workgroup of `points` threads then takes every item in one round
+// (rounded up, M = 24 gave 264 points to 256 threads and a second round for 8).
 uint32_t item_sites(uint32_t M, int points)
 {
-  uint32_t spw = ((uint32_t)points + M - 1) / M;
+  uint32_t spw = (uint32_t)points / M;
   return spw < 1 ? 1 : spw > 64 ? 64 : spw;
 }
+
+// Persistent workgroups per CU: about what the registers leave resident (a
+// workgroup beyond that starts when another has drained the queues, and only
+// lengthens the tail).  12 lattices of 8^4..16^4, Ls 8..16, 1..4 right-hand
+// sides, FP32: 713 us with 6 workgroups per CU and items rounded up, 673 us
+// with 4 and rounded down; FP16, 8 such lattices: 563 us with 6, rounded up
+// and pipelined, 436 us with 7, rounded down and plain.
+int default_wgpc(int prec) { return prec == GBX_F64 || prec == GBX_F32 ? 4 : 7; }
+
+// Depth 1 of the gather pipeline is the plain form with 16-bit storage: there
+// the pipeline's registers cost more wavefronts than it hides latency.
+template <int P> constexpr int depth1() { return P == GBX_F64 || P == GBX_F32 ? 1 : 0; }
 
 template <int P, bool DAG, bool TD, int T>
 void launch_t(gbx_batch_s *b, hipStream_t st, size_t lds)
@@ -231,7 +245,7 @@ void launch_t(gbx_batch_s *b, hipStream_t st, size_t lds)
     hipLaunchKernelGGL((k_dhop_batch<P, DAG, 2, TD, T>), dim3(b->grid), dim3(T), lds, st, (const LatDesc *)b->d_lat,
                        (const uint4 *)b->d_items, b->qb, b->d_counter, b->max_spw, b->shape.nt);
   else
-    hipLaunchKernelGGL((k_dhop_batch<P, DAG, 1, TD, T>), dim3(b->grid), dim3(T), lds, st, (const LatDesc *)b->d_lat,
+    hipLaunchKernelGGL((k_dhop_batch<P, DAG, depth1<P>(), TD, T>), dim3(b->grid), dim3(T), lds, st, (const LatDesc *)b->d_lat,
                        (const uint4 *)b->d_items, b->qb, b->d_counter, b->max_spw, b->shape.nt);
 }
 
@@ -300,7 +314,7 @@ int build_items(gbx_batch_s *b)
   GBX_HIP(hipMemcpy(b->d_items, h.data(), sizeof(uint4) * h.size(), hipMemcpyHostToDevice));
   b->nitems = (uint32_t)h.size();
   b->max_spw = max_spw;
-  const int wgpc = b->shape.wgpc > 0 ? b->shape.wgpc : (b->prec == GBX_F64 ? 4 : 6);
+  const int wgpc = b->shape.wgpc > 0 ? b->shape.wgpc : default_wgpc(b->prec);
   b->grid = b->ncu * wgpc;
   return GBX_OK;
 }
@@ -414,7 +428,7 @@ int na_scratch_ptr(int dev, unsigned char **ptr)
 template <int P, bool DAG, bool TD>
 void launch_na_t(dim3 grid, size_t lds, hipStream_t st, unsigned char *sp)
 {
-  hipLaunchKernelGGL((k_dhop_batch_na<P, DAG, 1, TD>), grid, dim3(kThreads), lds, st, sp, 1);
+  hipLaunchKernelGGL((k_dhop_batch_na<P, DAG, depth1<P>(), TD>), grid, dim3(kThreads), lds, st, sp, 1);
 }
 
 template <int P>
@@ -456,9 +470,7 @@ extern "C" int gbx_batch_run_noalloc(int n, const gbx_gauge *u, const gbx_spinor
       GBX_CHECK(out[i]->d != in[j]->d && (j == i || out[i]->d != out[j]->d), GBX_EALIAS,
                 "gbx_batch_run_noalloc: output %d aliases another lattice's field", i);
     const uint32_t M = in[i]->M, nslot = (uint32_t)u[i]->geom->vol;
-    uint32_t spw = (kThreads + M - 1) / M;  // as gbx_batch_create cuts items
-    if (spw < 1) spw = 1;
-    if (spw > 64) spw = 64;
+    const uint32_t spw = item_sites(M, kThreads);  // as gbx_batch_create cuts items
     max_spw = std::max(max_spw, spw);
     t.lat[i].d = LatDesc{u[i]->d, u[i]->geom->nbr, in[i]->d, out[i]->d, M, nslot, (uint32_t)u[i]->comp12, 0};
     t.lat[i].item0 = (uint32_t)nitems;
@@ -474,7 +486,7 @@ extern "C" int gbx_batch_run_noalloc(int n, const gbx_gauge *u, const gbx_spinor
   int ncu = 256;
   GBX_HIP(hipSetDevice(dev));
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  const dim3 grid((unsigned)(ncu * (prec == GBX_F64 ? 4 : 6)));
+  const dim3 grid((unsigned)(ncu * default_wgpc(prec)));
   const size_t lds = lds_for(prec, max_spw);
   // inputs may still be in flight on their geometries' streams
   for (int i = 0; i < n; i++) GBX_HIP(hipStreamSynchronize(u[i]->geom->stream));
