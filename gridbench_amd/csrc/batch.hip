@@ -230,13 +230,8 @@ uint32_t item_sites(uint32_t M, int points)
 // workgroup beyond that starts when another has drained the queues, and only
 // lengthens the tail).  12 lattices of 8^4..16^4, Ls 8..16, 1..4 right-hand
 // sides, FP32: 713 us with 6 workgroups per CU and items rounded up, 673 us
-// with 4 and rounded down; FP16, 8 such lattices: 563 us with 6, rounded up
-// and pipelined, 436 us with 7, rounded down and plain.
-int default_wgpc(int prec) { return prec == GBX_F64 || prec == GBX_F32 ? 4 : 7; }
-
-// Depth 1 of the gather pipeline is the plain form with 16-bit storage: there
-// the pipeline's registers cost more wavefronts than it hides latency.
-template <int P> constexpr int depth1() { return P == GBX_F64 || P == GBX_F32 ? 1 : 0; }
+// with 4 and rounded down; FP16, 8 such lattices: 402 us with 7, 385 us with 5.
+int default_wgpc(int prec) { return prec == GBX_F64 || prec == GBX_F32 ? 4 : 5; }
 
 template <int P, bool DAG, bool TD, int T>
 void launch_t(gbx_batch_s *b, hipStream_t st, size_t lds)
@@ -245,7 +240,7 @@ void launch_t(gbx_batch_s *b, hipStream_t st, size_t lds)
     hipLaunchKernelGGL((k_dhop_batch<P, DAG, 2, TD, T>), dim3(b->grid), dim3(T), lds, st, (const LatDesc *)b->d_lat,
                        (const uint4 *)b->d_items, b->qb, b->d_counter, b->max_spw, b->shape.nt);
   else
-    hipLaunchKernelGGL((k_dhop_batch<P, DAG, depth1<P>(), TD, T>), dim3(b->grid), dim3(T), lds, st, (const LatDesc *)b->d_lat,
+    hipLaunchKernelGGL((k_dhop_batch<P, DAG, 1, TD, T>), dim3(b->grid), dim3(T), lds, st, (const LatDesc *)b->d_lat,
                        (const uint4 *)b->d_items, b->qb, b->d_counter, b->max_spw, b->shape.nt);
 }
 
@@ -428,7 +423,7 @@ int na_scratch_ptr(int dev, unsigned char **ptr)
 template <int P, bool DAG, bool TD>
 void launch_na_t(dim3 grid, size_t lds, hipStream_t st, unsigned char *sp)
 {
-  hipLaunchKernelGGL((k_dhop_batch_na<P, DAG, depth1<P>(), TD>), grid, dim3(kThreads), lds, st, sp, 1);
+  hipLaunchKernelGGL((k_dhop_batch_na<P, DAG, 1, TD>), grid, dim3(kThreads), lds, st, sp, 1);
 }
 
 template <int P>

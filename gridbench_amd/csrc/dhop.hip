@@ -133,9 +133,8 @@ bool dhop_lookup_cfg(const std::string &sig, gbx_kcfg *c)
 //    otherwise, where the links of more sites are staged together; with one
 //    or two sites in a wavefront, a larger workgroup if it idles fewer lanes.
 //  * pf: the gather pipeline pays for its registers (FP64 2 wavefronts a SIMD
-//    instead of 4, FP32 5 instead of 8) except where the whole grid is resident
-//    in one round without it and not with it, and with 16-bit storage once
-//    the grid fills the card.
+//    instead of 4, FP32 5 instead of 8, 16-bit 6 instead of 7 or 8) except
+//    where the whole grid is resident in one round without it and not with it.
 dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
 {
   const bool f64 = in->prec == GBX_F64, f32 = in->prec == GBX_F32, f16 = !f64 && !f32;
@@ -160,7 +159,7 @@ dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
         }
       }
   } else if (M > 64) {
-    threads = f16 && M <= 85 ? 256 : 128;
+    threads = f16 ? 256 : 128;
     spw = sites(threads, M);
   } else {
     threads = f64 || (f32 && M >= 8 && pts <= (1u << 20)) || (f32 && pts <= 50000) ? 64 : 256;
@@ -176,7 +175,7 @@ dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
   c.mc = mc == M ? 0 : (int)mc;
   if (f64) c.pf = waves > 2048 && waves <= (M < 16 ? 3584u : 3072u) ? 0 : M <= 24 ? 1 : 2;
   else if (f32) c.pf = M <= 16 && waves > 5120 && waves <= 8192 ? 0 : M <= 24 ? 1 : 2;
-  else c.pf = waves <= 2048 ? 2 : 0;
+  else c.pf = M <= 64 && waves > 6144 && waves <= (in->prec == GBX_F16 ? 8192u : 7168u) ? 0 : 1;
   c.axpby_pf = true;
   c.wgpc = 0;
   c.cblk = 0;

@@ -20,43 +20,76 @@ template <bool DAG, int DIR> struct LegProj {
   static constexpr int value = DAG ? DIR : (DIR ^ 4);
 };
 
-// v[2*(sp*3+c) + {0,1}] = re/im of spin sp colour c of the neighbour spinor.
+// Sums and differences of a neighbour spinor's reals, real 2*(sp*3+c) + {0,1}
+// = re/im of spin sp colour c: of an array in the arithmetic type, ...
+template <typename A> struct Reals {
+  const A *v;
+  __device__ __forceinline__ A add(int i, int j) const { return v[i] + v[j]; }
+  __device__ __forceinline__ A sub(int i, int j) const { return v[i] - v[j]; }
+};
+
+// ... or of 16-bit chunks as they were loaded.  FP16: one v_fma_mix_f32 (a * 1
+// + b with both read as halves of a register), which takes the place of two
+// conversions and an addition; `one` is 1.0f the compiler cannot fold.  Both
+// round the exact sum once.
+template <int P> struct RawReals {
+  typename Traits<P>::vec c[Traits<P>::NCH];
+  float one;
+  __device__ __forceinline__ float real(int i) const { return (float)c[i >> 3][i & 7]; }
+  __device__ __forceinline__ float add(int i, int j) const
+  {
+    if constexpr (P == GBX_F16) return __builtin_fmaf(real(i), one, real(j));
+    else return real(i) + real(j);
+  }
+  __device__ __forceinline__ float sub(int i, int j) const
+  {
+    if constexpr (P == GBX_F16) return __builtin_fmaf(real(i), one, -real(j));
+    else return real(i) - real(j);
+  }
+};
+
 // h[0..2] = upper half-spinor row 0, h[3..5] = row 1 (re in hr, im in hi).
-template <int K, typename A>
-__device__ __forceinline__ void project(const A *v, A *hr, A *hi)
+template <int K, typename V, typename A>
+__device__ __forceinline__ void project_from(const V &v, A *hr, A *hi)
 {
-#define PR(sp, c) v[2 * ((sp) * 3 + (c))]
-#define PI(sp, c) v[2 * ((sp) * 3 + (c)) + 1]
+#define PR(sp, c) (2 * ((sp) * 3 + (c)))
+#define PI(sp, c) (2 * ((sp) * 3 + (c)) + 1)
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     if (K == PXP) {  // h0 = p0 + i p3, h1 = p1 + i p2
-      hr[c] = PR(0, c) - PI(3, c); hi[c] = PI(0, c) + PR(3, c);
-      hr[3 + c] = PR(1, c) - PI(2, c); hi[3 + c] = PI(1, c) + PR(2, c);
+      hr[c] = v.sub(PR(0, c), PI(3, c)); hi[c] = v.add(PI(0, c), PR(3, c));
+      hr[3 + c] = v.sub(PR(1, c), PI(2, c)); hi[3 + c] = v.add(PI(1, c), PR(2, c));
     } else if (K == PYP) {  // h0 = p0 - p3, h1 = p1 + p2
-      hr[c] = PR(0, c) - PR(3, c); hi[c] = PI(0, c) - PI(3, c);
-      hr[3 + c] = PR(1, c) + PR(2, c); hi[3 + c] = PI(1, c) + PI(2, c);
+      hr[c] = v.sub(PR(0, c), PR(3, c)); hi[c] = v.sub(PI(0, c), PI(3, c));
+      hr[3 + c] = v.add(PR(1, c), PR(2, c)); hi[3 + c] = v.add(PI(1, c), PI(2, c));
     } else if (K == PZP) {  // h0 = p0 + i p2, h1 = p1 - i p3
-      hr[c] = PR(0, c) - PI(2, c); hi[c] = PI(0, c) + PR(2, c);
-      hr[3 + c] = PR(1, c) + PI(3, c); hi[3 + c] = PI(1, c) - PR(3, c);
+      hr[c] = v.sub(PR(0, c), PI(2, c)); hi[c] = v.add(PI(0, c), PR(2, c));
+      hr[3 + c] = v.add(PR(1, c), PI(3, c)); hi[3 + c] = v.sub(PI(1, c), PR(3, c));
     } else if (K == PTP) {  // h0 = p0 + p2, h1 = p1 + p3
-      hr[c] = PR(0, c) + PR(2, c); hi[c] = PI(0, c) + PI(2, c);
-      hr[3 + c] = PR(1, c) + PR(3, c); hi[3 + c] = PI(1, c) + PI(3, c);
+      hr[c] = v.add(PR(0, c), PR(2, c)); hi[c] = v.add(PI(0, c), PI(2, c));
+      hr[3 + c] = v.add(PR(1, c), PR(3, c)); hi[3 + c] = v.add(PI(1, c), PI(3, c));
     } else if (K == PXM) {  // h0 = p0 - i p3, h1 = p1 - i p2
-      hr[c] = PR(0, c) + PI(3, c); hi[c] = PI(0, c) - PR(3, c);
-      hr[3 + c] = PR(1, c) + PI(2, c); hi[3 + c] = PI(1, c) - PR(2, c);
+      hr[c] = v.add(PR(0, c), PI(3, c)); hi[c] = v.sub(PI(0, c), PR(3, c));
+      hr[3 + c] = v.add(PR(1, c), PI(2, c)); hi[3 + c] = v.sub(PI(1, c), PR(2, c));
     } else if (K == PYM) {  // h0 = p0 + p3, h1 = p1 - p2
-      hr[c] = PR(0, c) + PR(3, c); hi[c] = PI(0, c) + PI(3, c);
-      hr[3 + c] = PR(1, c) - PR(2, c); hi[3 + c] = PI(1, c) - PI(2, c);
+      hr[c] = v.add(PR(0, c), PR(3, c)); hi[c] = v.add(PI(0, c), PI(3, c));
+      hr[3 + c] = v.sub(PR(1, c), PR(2, c)); hi[3 + c] = v.sub(PI(1, c), PI(2, c));
     } else if (K == PZM) {  // h0 = p0 - i p2, h1 = p1 + i p3
-      hr[c] = PR(0, c) + PI(2, c); hi[c] = PI(0, c) - PR(2, c);
-      hr[3 + c] = PR(1, c) - PI(3, c); hi[3 + c] = PI(1, c) + PR(3, c);
+      hr[c] = v.add(PR(0, c), PI(2, c)); hi[c] = v.sub(PI(0, c), PR(2, c));
+      hr[3 + c] = v.sub(PR(1, c), PI(3, c)); hi[3 + c] = v.add(PI(1, c), PR(3, c));
     } else {  // PTM: h0 = p0 - p2, h1 = p1 - p3
-      hr[c] = PR(0, c) - PR(2, c); hi[c] = PI(0, c) - PI(2, c);
-      hr[3 + c] = PR(1, c) - PR(3, c); hi[3 + c] = PI(1, c) - PI(3, c);
+      hr[c] = v.sub(PR(0, c), PR(2, c)); hi[c] = v.sub(PI(0, c), PI(2, c));
+      hr[3 + c] = v.sub(PR(1, c), PR(3, c)); hi[3 + c] = v.sub(PI(1, c), PI(3, c));
     }
   }
 #undef PR
 #undef PI
+}
+
+template <int K, typename A>
+__device__ __forceinline__ void project(const A *v, A *hr, A *hi)
+{
+  project_from<K>(Reals<A>{v}, hr, hi);
 }
 
 // The reference's arithmetic for U x chi: every complex product
@@ -87,34 +120,16 @@ __device__ __forceinline__ void su3_mul_exact(const A *U, const A *hr, const A *
 }
 
 // u[sp*3+i] = sum_j U[i][j] h[sp*3+j]; U row-major complex, 18 reals.
-// MUL_CHAIN (FP64 and FP32 storage): one multiply + five fused multiply-adds
-// per real output (72 ops per leg, 840 VALU ops per 5D site instead of 1032
-// for the mul/fma/add form the compiler derives from the plain expression).
-// MUL_PLAIN (16-bit storage): the plain expression, whose register schedule
-// keeps those kernels free of spills.  MUL_EXACT: the reference's rounding.
-enum { MUL_PLAIN = 0, MUL_CHAIN = 1, MUL_EXACT = 2 };
+// MUL_CHAIN: one multiply + five fused multiply-adds per real output (72 ops
+// per leg, 840 VALU ops per 5D site instead of 1032 for the mul/fma/add form
+// the compiler derives from the plain expression).  MUL_EXACT: the
+// reference's rounding.
+enum { MUL_CHAIN = 0, MUL_EXACT = 1 };
 template <int MUL, typename A>
 __device__ __forceinline__ void su3_mul(const A *U, const A *hr, const A *hi, A *ur, A *ui)
 {
   if constexpr (MUL == MUL_EXACT) {
     su3_mul_exact(U, hr, hi, ur, ui);
-    return;
-  }
-  if constexpr (MUL == MUL_PLAIN) {
-#pragma unroll
-    for (int sp = 0; sp < 2; sp++)
-#pragma unroll
-      for (int i = 0; i < 3; i++) {
-        A re = U[(i * 3) * 2] * hr[sp * 3] - U[(i * 3) * 2 + 1] * hi[sp * 3];
-        A im = U[(i * 3) * 2] * hi[sp * 3] + U[(i * 3) * 2 + 1] * hr[sp * 3];
-#pragma unroll
-        for (int j = 1; j < 3; j++) {
-          re += U[(i * 3 + j) * 2] * hr[sp * 3 + j] - U[(i * 3 + j) * 2 + 1] * hi[sp * 3 + j];
-          im += U[(i * 3 + j) * 2] * hi[sp * 3 + j] + U[(i * 3 + j) * 2 + 1] * hr[sp * 3 + j];
-        }
-        ur[sp * 3 + i] = re;
-        ui[sp * 3 + i] = im;
-      }
     return;
   }
 #pragma unroll
@@ -354,6 +369,75 @@ __device__ __forceinline__ void leg_apply(const A *v, const A *U, A *rr, A *ri)
   __builtin_amdgcn_s_setprio(0);
 }
 
+// An empty asm that reads and redefines the accumulators: every leg's
+// arithmetic is complete before the next leg's loads (otherwise the compiler
+// sinks all legs' arithmetic below all loads and keeps eight gathered
+// spinors live).
+template <typename A>
+__device__ __forceinline__ void pin_acc(A *rr, A *ri)
+{
+  asm volatile("" : "+v"(rr[0]), "+v"(rr[1]), "+v"(rr[2]), "+v"(rr[3]), "+v"(rr[4]), "+v"(rr[5]), "+v"(rr[6]),
+               "+v"(rr[7]), "+v"(rr[8]), "+v"(rr[9]), "+v"(rr[10]), "+v"(rr[11]));
+  asm volatile("" : "+v"(ri[0]), "+v"(ri[1]), "+v"(ri[2]), "+v"(ri[3]), "+v"(ri[4]), "+v"(ri[5]), "+v"(ri[6]),
+               "+v"(ri[7]), "+v"(ri[8]), "+v"(ri[9]), "+v"(ri[10]), "+v"(ri[11]));
+}
+
+// 16-bit storage: the legs work on the chunks as loaded (12 registers a leg
+// instead of 24), converted by the projection.  What bounds these kernels is
+// the VALU as much as the gathers: 24^4 x Ls16 FP16, converting on load and with
+// unchained products, took 1250 operations a point (190 of 243 us); 880 here,
+// 211 us.  BF16 keeps its conversions: 1075.  16^3x24 x Ls12 x 16 BF16: 777 ->
+// 659 us.
+template <int P>
+__device__ __forceinline__ void load_raw(const void *__restrict__ in, uint32_t nb, uint32_t M, uint32_t m, RawReals<P> &v)
+{
+  const typename Traits<P>::vec *p = (const typename Traits<P>::vec *)in + (uint64_t)nb * Traits<P>::NCH * M + m;
+#pragma unroll
+  for (int k = 0; k < Traits<P>::NCH; k++) v.c[k] = p[(uint64_t)k * M];
+}
+
+template <int P, bool DAG, int D>
+__device__ __forceinline__ void leg_raw(const RawReals<P> &v, const float *U, float *rr, float *ri)
+{
+  float hr[6], hi[6], ur[6], ui[6];
+  __builtin_amdgcn_s_setprio(1);
+  project_from<LegProj<DAG, D>::value>(v, hr, hi);
+  su3_mul<MUL_CHAIN>(U, hr, hi, ur, ui);
+  recon<LegProj<DAG, D>::value, D == 0>(ur, ui, rr, ri);
+  __builtin_amdgcn_s_setprio(0);
+}
+
+// PF legs are gathered ahead of the one being computed; the scheduling barrier
+// and the pinned accumulators keep the compiler from gathering (and holding)
+// more of them, or from sinking the arithmetic into the stores' branches.
+template <int P, bool DAG, int PF>
+__device__ __forceinline__ void dhop_site_raw(const void *__restrict__ in, const uint32_t *nb, uint32_t M, uint32_t m,
+                                              const float *U, float *rr, float *ri)
+{
+  float one = 1.0f;
+  if (P == GBX_F16) asm volatile("" : "+s"(one));
+  RawReals<P> v[PF + 1];
+#pragma unroll
+  for (int d = 0; d <= PF; d++) v[d].one = one;
+#pragma unroll
+  for (int d = 0; d < PF; d++) load_raw<P>(in, nb[d], M, m, v[d]);
+#define GBX_RLEG(D)                                                                \
+  if (D + PF < 8) load_raw<P>(in, nb[(D + PF) & 7], M, m, v[(D + PF) % (PF + 1)]); \
+  __builtin_amdgcn_sched_barrier(0);                                               \
+  leg_raw<P, DAG, D>(v[D % (PF + 1)], U + D * 18, rr, ri);                         \
+  pin_acc(rr, ri);                                                                 \
+  __builtin_amdgcn_sched_barrier(0);
+  GBX_RLEG(0)
+  GBX_RLEG(1)
+  GBX_RLEG(2)
+  GBX_RLEG(3)
+  GBX_RLEG(4)
+  GBX_RLEG(5)
+  GBX_RLEG(6)
+  GBX_RLEG(7)
+#undef GBX_RLEG
+}
+
 // Full 8-leg hopping term for (site with links U, neighbours nb[8], minor m).
 // PF = 0: gather and compute leg by leg.  PF = 1: the gather of leg d+1 is
 // issued before leg d is computed (two gather buffers in registers), which
@@ -366,8 +450,11 @@ __device__ __forceinline__ void dhop_site(const void *__restrict__ in, const uin
                                           typename Traits<P>::acc *ri)
 {
   typedef typename Traits<P>::acc A;
-  constexpr int CH = EXACT ? MUL_EXACT : (P == GBX_F64 || P == GBX_F32) ? MUL_CHAIN : MUL_PLAIN;
-  if (PF == 0) {
+  constexpr int CH = EXACT ? MUL_EXACT : MUL_CHAIN;
+  if constexpr (P == GBX_F16 || P == GBX_BF16) {
+    static_assert(!EXACT && !TD, "FP64 / FP32 forms");
+    dhop_site_raw<P, DAG, PF>(in, nb, M, m, U, rr, ri);
+  } else if (PF == 0) {
     A v[24];
 #define GBX_LEG(D, FIRST)                                                  \
     leg_load<P, DAG, D, TD>(in, nb[D], M, m, v);                           \
@@ -427,7 +514,7 @@ __device__ __forceinline__ void dhop_site_gp(const void *__restrict__ in, const 
                                              typename Traits<P>::acc *rr, typename Traits<P>::acc *ri)
 {
   typedef typename Traits<P>::acc A;
-  constexpr int CH = (P == GBX_F64 || P == GBX_F32) ? MUL_CHAIN : MUL_PLAIN;
+  constexpr int CH = MUL_CHAIN;
   if (PF == 0) {
     A v[24];
 #define GBX_LEG(D, FIRST)                                                                  \

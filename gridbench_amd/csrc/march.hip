@@ -70,19 +70,6 @@ __device__ __forceinline__ void lds_leg(const V *p, uint32_t cs, A *v)
 
 template <int P> constexpr int march_max_threads() { return P == GBX_F64 ? 256 : 512; }
 
-// An empty asm that reads and redefines the accumulators: every leg's
-// arithmetic is complete before the next leg's loads (otherwise the compiler
-// sinks all legs' arithmetic below all loads and keeps eight gathered
-// spinors live).
-template <typename A>
-__device__ __forceinline__ void pin_acc(A *rr, A *ri)
-{
-  asm volatile("" : "+v"(rr[0]), "+v"(rr[1]), "+v"(rr[2]), "+v"(rr[3]), "+v"(rr[4]), "+v"(rr[5]), "+v"(rr[6]),
-               "+v"(rr[7]), "+v"(rr[8]), "+v"(rr[9]), "+v"(rr[10]), "+v"(rr[11]));
-  asm volatile("" : "+v"(ri[0]), "+v"(ri[1]), "+v"(ri[2]), "+v"(ri[3]), "+v"(ri[4]), "+v"(ri[5]), "+v"(ri[6]),
-               "+v"(ri[7]), "+v"(ri[8]), "+v"(ri[9]), "+v"(ri[10]), "+v"(ri[11]));
-}
-
 template <int P, bool DAG, bool TD>
 __global__ void __launch_bounds__(march_max_threads<P>()) k_dhop_march(MarchArgs a)
 {
@@ -90,7 +77,7 @@ __global__ void __launch_bounds__(march_max_threads<P>()) k_dhop_march(MarchArgs
   typedef typename dev::Traits<P>::vec V;
   typedef typename dev::Traits<P>::st S;
   constexpr int NCH = dev::Traits<P>::NCH;
-  constexpr int CH = (P == GBX_F64 || P == GBX_F32) ? dev::MUL_CHAIN : dev::MUL_PLAIN;
+  constexpr int CH = dev::MUL_CHAIN;
   const int md = a.md, TS = a.e[md];
   // the three tile dimensions, ascending
   int td[3], n3 = 0;
@@ -249,7 +236,7 @@ __global__ void __launch_bounds__(march_max_threads<P>()) k_dhop_march(MarchArgs
         dev::leg_load<P, DAG, D, TD>(a.in, nbq[D], a.M, m, v);                                                         \
         dev::leg_apply<DAG, D, TD, FIRST, CH>(v, Uq + (D) * 18, rr, ri);                                               \
       }                                                                                                                \
-      pin_acc(rr, ri);                                                                                                 \
+      dev::pin_acc(rr, ri);                                                                                                 \
     }
     GBX_MLEG(0, true)
     GBX_MLEG(1, false)

@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(tile_max_threads(P, TD)) k_dhop_tile(TileArgs 
   // 12 chunks are padded to 13 so that 8 consecutive lanes' 16-byte reads
   // fall in distinct banks.
   constexpr int SW = NCH == 12 ? 13 : NCH;
-  constexpr int CH = (P == GBX_F64 || P == GBX_F32) ? dev::MUL_CHAIN : dev::MUL_PLAIN;
+  constexpr int CH = dev::MUL_CHAIN;
   const int e[4] = {a.ex, a.ey, a.ez, a.et};
   const int T = e[0] * e[1] * e[2] * e[3];
   extern __shared__ __align__(16) unsigned char smem[];
@@ -226,11 +226,26 @@ __global__ void __launch_bounds__(tile_max_threads(P, TD)) k_dhop_tile(TileArgs 
     const uint32_t ml = w - (uint32_t)i * mcc, m = m0 + ml;
     A rr[12], ri[12];
     A v[24];
+    float one = 1.0f;
+    if (P == GBX_F16) asm volatile("" : "+s"(one));
+    // (16-bit storage: the chunks as they are, converted by the projection.)
 #define GBX_TLEG(D, FIRST)                                                                                             \
     {                                                                                                                  \
       const int ln = sL[i * 8 + (D)];                                                                                  \
-      if (ln >= 0) {                                                                                                   \
-        lds_leg_load<P, DAG, D, TD>(sIn + ((uint32_t)ln * a.mc + ml) * SW, v);                                         \
+      const V *pl = sIn + ((uint32_t)ln * a.mc + ml) * SW;                                                             \
+      if constexpr (P == GBX_F16 || P == GBX_BF16) {                                                                   \
+        dev::RawReals<P> raw;                                                                                          \
+        raw.one = one;                                                                                                 \
+        if (ln >= 0) {                                                                                                 \
+          _Pragma("unroll") for (int k = 0; k < NCH; k++) raw.c[k] = pl[k];                                            \
+          dev::leg_raw<P, DAG, D>(raw, sU + (i * 8 + D) * 18, rr, ri);                                                 \
+        } else {                                                                                                       \
+          dev::load_raw<P>(a.in, sN[i * 8 + D], a.M, m, raw);                                                          \
+          dev::leg_raw<P, DAG, D>(raw, sU + (i * 8 + D) * 18, rr, ri);                                                 \
+        }                                                                                                              \
+        dev::pin_acc(rr, ri);                                                                                          \
+      } else if (ln >= 0) {                                                                                            \
+        lds_leg_load<P, DAG, D, TD>(pl, v);                                                                            \
         dev::leg_apply<DAG, D, TD, FIRST, CH>(v, sU + (i * 8 + D) * 18, rr, ri);                                       \
       } else {                                                                                                         \
         dev::leg_load<P, DAG, D, TD>(a.in, sN[i * 8 + D], a.M, m, v);                                                  \

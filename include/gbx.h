@@ -566,9 +566,8 @@ int gbx_batch_time(gbx_batch b, int nrep, double *usec);
 /* Work items and persistent workgroups of the launch. */
 int gbx_batch_info(gbx_batch b, uint64_t *items, int *workgroups);
 /* Launch shape of the persistent kernel, in gbx_kcfg fields: threads (256 */
-/* or 512 per workgroup), pf (gather pipeline depth 1 or 2; 1 is none with */
-/* 16-bit storage), wgpc (persistent workgroups per CU; 0 = 4 for FP64 and */
-/* FP32, 7 otherwise), nt                                                  */
+/* or 512 per workgroup), pf (gather pipeline depth 1 or 2), wgpc          */
+/* (persistent workgroups per CU; 0 = 4 for FP64 and FP32, 5 otherwise), nt */
 /* (streaming stores) and spw (the (site, minor) points a work item aims   */
 /* at: a lattice of minor extent M is cut into items of floor(spw / M)     */
 /* sites, 1 to 64).  gbx_batch_create starts at threads 256, pf 1,     */
