@@ -117,6 +117,7 @@ struct gbx_dslash_ctx_s {
   gbx_spinor sin = nullptr, sout = nullptr;
   int dims[4] = {0, 0, 0, 0}, Ls = 0, prec = -1;
   hipStream_t st = nullptr;  // table path; the fast path runs on its geometry's stream
+  HostRing ring;             // pinned staging of the host arrays
   int last_path = 0;
 };
 
@@ -225,8 +226,8 @@ int dslash_kernel_impl(gbx_dslash_ctx_s &c, int nrep, int nsimd, int dsimd, int 
     // The SoA kernel, once per replica of the dsimd-lane lattice.
     GBX_TRY(fast_objects(c, dims, (int)Ls, RefPrec<T>::prec));
     hipStream_t st = c.geom->stream;
-    GBX_HIP(hipMemcpyAsync(c.dU, U, nu, hipMemcpyHostToDevice, st));
-    GBX_HIP(hipMemcpyAsync(c.dIn, in, nf, hipMemcpyHostToDevice, st));
+    GBX_TRY(c.ring.upload(c.dU, U, nu, st));
+    GBX_TRY(c.ring.upload(c.dIn, in, nf, st));
     double total = 0.0;
     for (int nn = 0; nn < nsimd / dsimd; nn++) {
       gbx_ref_layout lay;
@@ -240,8 +241,7 @@ int dslash_kernel_impl(gbx_dslash_ctx_s &c, int nrep, int nsimd, int dsimd, int 
       total += us;
       GBX_TRY(ref_unpack_spinor_dev(c.sout, (T *)c.dOut, dsimd, lay));
     }
-    GBX_HIP(hipMemcpyAsync(out, c.dOut, nf, hipMemcpyDeviceToHost, st));
-    GBX_HIP(hipStreamSynchronize(st));
+    GBX_TRY(c.ring.download(out, c.dOut, nf, st));
     if (usec) *usec = total;
     c.last_path = 1;
     return GBX_OK;
@@ -250,10 +250,10 @@ int dslash_kernel_impl(gbx_dslash_ctx_s &c, int nrep, int nsimd, int dsimd, int 
   GBX_TRY(ensure(&c.dNbr, &c.nNbr, nt * 8));
   GBX_TRY(ensure(&c.dPrm, &c.nPrm, nt));
   hipStream_t st = c.st;
-  GBX_HIP(hipMemcpyAsync(c.dU, U, nu, hipMemcpyHostToDevice, st));
-  GBX_HIP(hipMemcpyAsync(c.dIn, in, nf, hipMemcpyHostToDevice, st));
-  GBX_HIP(hipMemcpyAsync(c.dNbr, nbr, nt * 8, hipMemcpyHostToDevice, st));
-  GBX_HIP(hipMemcpyAsync(c.dPrm, prm, nt, hipMemcpyHostToDevice, st));
+  GBX_TRY(c.ring.upload(c.dU, U, nu, st));
+  GBX_TRY(c.ring.upload(c.dIn, in, nf, st));
+  GBX_TRY(c.ring.upload(c.dNbr, nbr, nt * 8, st));
+  GBX_TRY(c.ring.upload(c.dPrm, prm, nt, st));
   const uint64_t nthr = n5 * (uint64_t)nsimd;
   const dim3 grid((unsigned)((nthr + 255) / 256)), block(256);
   auto launch = [&]() -> int {
@@ -269,8 +269,7 @@ int dslash_kernel_impl(gbx_dslash_ctx_s &c, int nrep, int nsimd, int dsimd, int 
     return GBX_OK;
   };
   GBX_TRY(timed_reps(nrep, st, launch, usec));
-  GBX_HIP(hipMemcpyAsync(out, c.dOut, nf, hipMemcpyDeviceToHost, st));
-  GBX_HIP(hipStreamSynchronize(st));
+  GBX_TRY(c.ring.download(out, c.dOut, nf, st));
   c.last_path = 2;
   return GBX_OK;
 }
@@ -278,6 +277,7 @@ int dslash_kernel_impl(gbx_dslash_ctx_s &c, int nrep, int nsimd, int dsimd, int 
 void ctx_release(gbx_dslash_ctx_s &c)
 {
   if (c.st) (void)hipStreamSynchronize(c.st);
+  c.ring.release();
   for (void *p : {c.dU, c.dIn, c.dOut, c.dNbr, c.dPrm}) (void)hipFree(p);
   c.dU = c.dIn = c.dOut = c.dNbr = c.dPrm = nullptr;
   c.nU = c.nIn = c.nOut = c.nNbr = c.nPrm = 0;

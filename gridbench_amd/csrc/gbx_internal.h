@@ -151,6 +151,24 @@ int require_chiral(const char *what, const gbx_spinor_s *a, const gbx_spinor_s *
 void geom_retain(gbx_geom_s *g);
 void geom_release(gbx_geom_s *g);
 
+// Pinned buffers for copies of pageable host arrays (hostcopy.cpp).  One owner
+// uses it at a time; kSlots * kBytes of pinned memory once a copy of at least
+// kSmall went through it, until release().
+struct HostRing {
+  static constexpr int kSlots = 4;
+  static constexpr size_t kBytes = 4 << 20, kSmall = 1 << 20;
+  void *buf[kSlots] = {};
+  hipEvent_t ev[kSlots] = {};
+  bool used[kSlots] = {};
+  int next = 0;
+  int upload(void *dst, const void *src, size_t n, hipStream_t st);
+  int download(void *dst, const void *src, size_t n, hipStream_t st);
+  void release();
+
+ private:
+  int prepare();
+};
+
 // Scratch buffer reused by uploads/downloads (grows on demand, per geometry
 // stream; freed with the library's cached allocations at exit).
 int staging_buffer(size_t bytes, void **ptr);
