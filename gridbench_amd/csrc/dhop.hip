@@ -302,6 +302,10 @@ int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in,
       a.Ls = (uint32_t)in->Ls;
       epi = EPI_S5;
     }
+    if (s5 == dhop_fuse::MOOEE && dhop_s5inv_fits(in, c)) {
+      a.lds = std::max(a.lds, (size_t)c.threads * 16 * (u->prec == GBX_F64 ? 6 : 3));
+      epi = EPI_S5X;
+    }
     if (s5 == dhop_fuse::MOOEE_INV) {
       GBX_CHECK(dhop_s5inv_fits(in, c), GBX_EUNSUPPORTED, "dhop: Mooee^-1 does not fit this launch shape");
       a.lds = std::max(a.lds, (size_t)c.threads * 12 * (u->prec == GBX_F64 ? 8 : 4));

@@ -5,8 +5,8 @@
 // The hopping kernels are bound by their gathers (dhop.hip), so what an
 // epilogue adds is the traffic of its own operands: D = Mooee - Dhop / 2 at
 // 24^4 x Ls16 FP64 took 836 us for Dhop and 491 us for a pass over three
-// fields that adds Mooee; in one kernel it takes 870 us (FP32: 627 -> 424 us),
-// 57 us over Dhop alone for a third field to read.  The even-odd operator's
+// fields that adds Mooee; in one kernel it takes 863 us (FP32: 627 -> 424 us),
+// 50 us over Dhop alone for a third field to read.  The even-odd operator's
 // Mooee^-1 DhopOE (16^4 x Ls12 FP32: 29 + 16 us as two kernels) saves the pass
 // over the half lattice too; the domain-wall solve there went from 26.4 to
 // 22.2 ms with both.
@@ -33,6 +33,10 @@ void pick_epi(int epi, bool dag, bool td, bool red, int pf, const LaunchArgs &a)
     if (dag) pick_pf<P, true, C12, EPI_S5, false, false>(pf, a);
     else if (red) pick_pf<P, false, C12, EPI_S5, false, true>(pf, a);
     else pick_pf<P, false, C12, EPI_S5, false, false>(pf, a);
+  } else if (epi == EPI_S5X) {
+    if (dag) pick_pf<P, true, C12, EPI_S5X, false, false>(pf, a);
+    else if (red) pick_pf<P, false, C12, EPI_S5X, false, true>(pf, a);
+    else pick_pf<P, false, C12, EPI_S5X, false, false>(pf, a);
   } else {
     if constexpr (P == GBX_F64 || P == GBX_F32) {
       if (td) {

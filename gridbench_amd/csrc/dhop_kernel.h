@@ -14,7 +14,8 @@ enum {
   EPI_STORE = 0,  // out = Dhop in
   EPI_AXPBY = 1,  // out = alpha c + beta Dhop in
   EPI_S5 = 2,     // out = Mooee c + beta Dhop in  (the adjoint of Mooee for DAG)
-  EPI_S5INV = 3   // out = Mooee^-1 Dhop in  (the adjoint for DAG)
+  EPI_S5INV = 3,  // out = Mooee^-1 Dhop in  (the adjoint for DAG)
+  EPI_S5X = 4     // EPI_S5 in workgroups that hold whole columns of slices
 };
 
 template <typename A> struct Epi {
@@ -58,6 +59,68 @@ __device__ __forceinline__ void store_s5(void *__restrict__ out, const void *__r
       if (RED) norm += (double)v[j] * (double)v[j];
     }
     dev::store_chunk<P, A>(out, base + (uint64_t)k * M + m, v, nt);
+  }
+}
+
+// store_s5 for a workgroup that holds whole (site, right-hand side) columns of
+// Ls slices, one point per thread: each thread reads its own slice of c only
+// and takes the neighbour slices from LDS, a chirality at a time (16-bit
+// fields all three chunks at once).  Half the loads of store_s5 and fewer
+// registers (FP32 72 instead of 81, 73 instead of 96 with the norm: 7 or 6
+// wavefronts a SIMD instead of 5).  What bounds the kernel is still the legs' gathers: 24^4 x
+// Ls16 FP64 869 -> 863 us, the domain-wall solve at 16^4 x Ls12, FP32 inner,
+// 16.40 -> 16.28 ms.  Every thread calls it; `w` is the point's index in the
+// workgroup, s its slice, `active`
+// whether it has one.
+template <int P, bool DAG, bool RED>
+__device__ __forceinline__ void store_s5x(void *__restrict__ out, const void *__restrict__ c, uint32_t q, uint32_t M, uint32_t m,
+                                          const Epi<typename dev::Traits<P>::acc> &e, uint32_t w, uint32_t s, bool active,
+                                          unsigned char *smem, typename dev::Traits<P>::acc *rr,
+                                          typename dev::Traits<P>::acc *ri, bool nt, double &norm)
+{
+  typedef typename dev::Traits<P>::acc A;
+  typedef typename dev::Traits<P>::vec V;
+  constexpr int NCH = dev::Traits<P>::NCH, R = dev::Traits<P>::R, G = R == 8 ? NCH : NCH / 2;
+  V *sx = (V *)smem;  // [G][threads]
+  const uint64_t base = (uint64_t)q * NCH * M + m;
+  const uint32_t th = blockDim.x;
+  const uint32_t wdn = s == 0 ? w + e.Ls - 1 : w - 1, wup = s == e.Ls - 1 ? w - (e.Ls - 1) : w + 1;
+  const A cdn = s == 0 ? e.mass : (A)-1, cup = s == e.Ls - 1 ? e.mass : (A)-1;
+#pragma unroll
+  for (int k0 = 0; k0 < NCH; k0 += G) {
+    V own[G];
+    __builtin_amdgcn_sched_barrier(0);  // c's chunks are not held across the legs
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < G; k++) own[k] = ((const V *)c)[base + (uint64_t)(k0 + k) * M];
+    }
+    __syncthreads();  // the links, or the other chirality, are no longer read
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < G; k++) sx[k * th + w] = own[k];
+    }
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < G; k++) {
+        __builtin_amdgcn_sched_barrier(0);  // one chunk's reals at a time
+        const int r0 = (k0 + k) * R;
+        const bool has_dn = DAG ? r0 + R > 12 : r0 < 12, has_up = DAG ? r0 < 12 : r0 + R > 12;
+        V dn, up;
+        A v[R];
+        if (has_dn) dn = sx[k * th + wdn];
+        if (has_up) up = sx[k * th + wup];
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+          const int r = r0 + j;
+          const bool down = (r < 12) != DAG;
+          const A acc = e.d * (A)own[k][j] + (down ? cdn : cup) * (A)(down ? dn[j] : up[j]);
+          v[j] = acc + e.beta * ((r & 1) ? ri[r >> 1] : rr[r >> 1]);
+          if (RED) norm += (double)v[j] * (double)v[j];
+        }
+        dev::store_chunk<P, A>(out, base + (uint64_t)(k0 + k) * M, v, nt);
+      }
+    }
   }
 }
 
@@ -123,6 +186,50 @@ __device__ __forceinline__ void s5_inverse(const Epi<A> &e, uint32_t w, uint32_t
   }
 }
 
+// A point's site and minor index once more: not kept in registers across the
+// legs.
+__device__ __forceinline__ void again(uint32_t &w, uint32_t mcc, uint32_t &sl, uint32_t &m)
+{
+  asm volatile("" : "+v"(w));
+  sl = w / mcc;
+  m = w - sl * mcc;
+}
+
+// out = alpha c + beta r of one point and its |out|^2, a chunk at a time: with
+// all 24 results and their squares in registers together the 16-bit forms need
+// more than the plain kernel's 80 and lose a wavefront of six.  CG at 16^3x24
+// x Ls8, FP16 inner: 13.6 -> 13.1 ms.
+template <int P>
+__device__ __forceinline__ void store_axpby_norm(void *__restrict__ out, const void *__restrict__ c, uint32_t q, uint32_t M,
+                                                 uint32_t m, const Epi<typename dev::Traits<P>::acc> &e,
+                                                 typename dev::Traits<P>::acc *rr, typename dev::Traits<P>::acc *ri, bool nt,
+                                                 double &norm)
+{
+  typedef typename dev::Traits<P>::acc A;
+  typedef typename dev::Traits<P>::vec V;
+  constexpr int NCH = dev::Traits<P>::NCH, R = dev::Traits<P>::R, G = NCH < 6 ? NCH : NCH / 2;
+  const uint64_t base = (uint64_t)q * NCH * M + m;
+#pragma unroll
+  for (int k0 = 0; k0 < NCH; k0 += G) {
+    V own[G];
+    __builtin_amdgcn_sched_barrier(0);  // c's chunks are not held across the legs
+#pragma unroll
+    for (int k = 0; k < G; k++) own[k] = ((const V *)c)[base + (uint64_t)(k0 + k) * M];
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+      __builtin_amdgcn_sched_barrier(0);
+      A v[R];
+#pragma unroll
+      for (int j = 0; j < R; j++) {
+        const int r = (k0 + k) * R + j;
+        v[j] = e.alpha * (A)own[k][j] + e.beta * ((r & 1) ? ri[r >> 1] : rr[r >> 1]);
+        norm += (double)v[j] * (double)v[j];
+      }
+      dev::store_chunk<P, A>(out, base + (uint64_t)(k0 + k) * M, v, nt);
+    }
+  }
+}
+
 // Sum over the workgroup in a fixed order (at most 16 wavefronts).
 __device__ __forceinline__ double block_sum(double a)
 {
@@ -176,27 +283,43 @@ __global__ void __launch_bounds__(PF ? 256 : 1024)
   dev::stage_links<P, C12>(gauge, nbr, q0, nsl, sU, sN);
 
   const uint32_t items = nsl * mcc;
-  if constexpr (EPI == EPI_S5INV) {  // one point per thread, whole columns
-    const uint32_t w = threadIdx.x, sl = w / mcc, m = w - sl * mcc;
+  if constexpr (EPI == EPI_S5INV || EPI == EPI_S5X) {  // one point per thread, whole columns
+    uint32_t w = threadIdx.x, sl = w / mcc, m = w - sl * mcc;
     const bool active = w < items;
     A rr[12], ri[12];
-    if (active) dev::dhop_site<P, DAG, PF, EXACT, TD>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
+    if (active) {
+      dev::dhop_site<P, DAG, PF, EXACT, TD>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
+      dev::pin_acc(rr, ri);
+    }
+    again(w, mcc, sl, m);
+    if constexpr (EPI == EPI_S5X) {
+      double norm = 0.0;
+      store_s5x<P, DAG, RED>(out, center, q0 + sl, M, m, e, w, m % e.Ls, active, smem, rr, ri, nt != 0, norm);
+      if constexpr (RED) {
+        norm = block_sum(norm);
+        if (threadIdx.x == 0) e.partial[L] = norm;
+      }
+      return;
+    }
     s5_inverse<DAG>(e, w, m % e.Ls, active, smem, rr, ri);
     if (active) dev::store_site<P, false>(out, nullptr, q0 + sl, M, m, rr, ri, (A)0, (A)1, nt != 0);
     return;
   }
   double norm = 0.0;
   for (uint32_t w = threadIdx.x; w < items; w += blockDim.x) {
-    const uint32_t sl = w / mcc, m = m0 + (w - sl * mcc);
+    uint32_t sl = w / mcc, m = m0 + (w - sl * mcc);
     A rr[12], ri[12];
     if constexpr (GP) dev::dhop_site_gp<P, DAG, PF>(in, sN + sl * 8, M, m, ghost0, sU + sl * 8 * 18, rr, ri);
     else dev::dhop_site<P, DAG, PF, EXACT, TD>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
-    if constexpr (EPI == EPI_S5) store_s5<P, DAG, RED>(out, center, q0 + sl, M, m, e, rr, ri, nt != 0, norm);
-    else dev::store_site<P, EPI == EPI_AXPBY>(out, center, q0 + sl, M, m, rr, ri, e.alpha, e.beta, nt != 0);
-    if constexpr (RED && EPI != EPI_S5) {
-#pragma unroll
-      for (int i = 0; i < 12; i++) norm += (double)rr[i] * (double)rr[i] + (double)ri[i] * (double)ri[i];
+    if constexpr (EPI == EPI_AXPBY && RED) {
+      uint32_t w2 = w;
+      dev::pin_acc(rr, ri);
+      again(w2, mcc, sl, m);
+      m += m0;
     }
+    if constexpr (EPI == EPI_S5) store_s5<P, DAG, RED>(out, center, q0 + sl, M, m, e, rr, ri, nt != 0, norm);
+    else if constexpr (RED) store_axpby_norm<P>(out, center, q0 + sl, M, m, e, rr, ri, nt != 0, norm);
+    else dev::store_site<P, EPI == EPI_AXPBY>(out, center, q0 + sl, M, m, rr, ri, e.alpha, e.beta, nt != 0);
   }
   if constexpr (RED) {
     norm = block_sum(norm);
