@@ -10,27 +10,32 @@
 //   r_in = s * r with s = sqrt(N) / |r|  (unit-RMS entries: safe for FP16)
 //   e = inner_solve(M_lo^dag M_lo e = r_in) to |r_in - ...| <= inner_tol |r_in|
 //   x += e / s          (reliable update of x in FP64)
-// Inner CG: vectors e, r in FP32; p and A p in the low storage precision of
+// Inner CG: vectors e, r in FP32; p and t = M p in the low storage precision of
 // the inner gauge field (FP32, FP16 or BF16), which is what the low-precision
 // hopping kernel reads and writes; every arithmetic operation in FP32; dots
 // and norms in FP64 with deterministic reductions.  With A = M^dag M one
 // iteration is
 //   t = M p, and <p, A p> = |t|^2 summed by the kernel that writes t
-//   Ap = M^dag t
-//   k_cg_r:  r -= a Ap, |r|^2          (a = |r_old|^2 / |t|^2)
-//   k_cg_ep: e += a p, p = r + b p     (b = |r|^2 / |r_old|^2)
-// The scalars stay on the device: every workgroup sums the partial sums it
-// needs itself, in one order, so no kernel waits for the host.  The host
+//   k_cg_alpha:  a = |r_old|^2 / |t|^2
+//   r -= a M^dag t and |r|^2 in the epilogue of the kernel that forms M^dag t,
+//     which is never stored
+//   k_cg_ep: p = r + b p (b = |r|^2 / |r_old|^2), and every other iteration
+//     e += a' p' + a p for the last two
+// The scalars stay on the device, so no kernel waits for the host.  The host
 // enqueues a few iterations ahead and learns of convergence from a word the
 // device writes to its memory; what was enqueued beyond it does nothing.
-// (With the two sums read back by the host, a dot product over p and A p, and
-// r, e and p updated in passes that read r twice and p three times, an
-// iteration at 16^3x24 x Ls8, FP16 inner, took 307 us, 90 of them idle; it
-// now takes 190 us, none of them idle: 51 us for each hop, 34 us (5.5 TB/s) for
-// k_cg_r and 48 us (6.3 TB/s) for k_cg_ep.)
+// An iteration at 16^3x24 x Ls8, FP16 inner, takes 137 us with no gaps: 42 us
+// for M p, 55 us for M^dag t with the update of r, 5 us for k_cg_alpha, and 23
+// or 45 us for k_cg_ep (6 TB/s).  It took 307 us with the two sums read back by
+// the host and the updates in passes of their own, and 163 us with the scalars
+// on the device but M^dag t stored and read again (30 us) and e updated each
+// time (42 us): 13.6 -> 12.0 ms a solve; domain-wall solve 16^4 x Ls12, FP32
+// inner: 16.3 -> 15.2 ms.  The partial sums are summed where they are needed
+// up to kPlain of them, which costs a reader 2 us; a pass of its own takes 5.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <mutex>
 #include <vector>
 
 #include "dhop_dev.h"
@@ -40,7 +45,7 @@ namespace {
 
 // Workgroups and threads of a pass over a field; partial sums beyond kPlain
 // are folded into kFold first.
-constexpr int kRB = 1024, kRT = 256, kPlain = 4096, kFold = 256;
+constexpr int kRB = 1024, kRT = 256, kAT = 1024, kPlain = 8192, kFold = 256;
 
 template <int P> struct Pt {
   typedef typename dev::Traits<P>::acc A;
@@ -61,10 +66,11 @@ __device__ __forceinline__ void store_pt(void *b, uint64_t q, uint32_t M, uint32
   for (int k = 0; k < Pt<P>::NCH; k++) dev::store_chunk<P, A>(b, (q * Pt<P>::NCH + k) * M + m, v + k * Pt<P>::R, false);
 }
 
-// Sum over the workgroup of kRT threads in a fixed order; every thread gets it.
+// Sum over the workgroup of T threads in a fixed order; every thread gets it.
+template <int T = kRT>
 __device__ __forceinline__ double bsum(double a)
 {
-  __shared__ double sh[kRT / 64];
+  __shared__ double sh[T / 64];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
   __syncthreads();  // an earlier sum has been read
@@ -72,24 +78,27 @@ __device__ __forceinline__ double bsum(double a)
   __syncthreads();
   double t = 0.0;
 #pragma unroll
-  for (int i = 0; i < kRT / 64; i++) t += sh[i];
+  for (int i = 0; i < T / 64; i++) t += sh[i];
   return t;
 }
 
 // Sum of n partial sums, by every workgroup on its own.
+template <int T = kRT>
 __device__ __forceinline__ double sum_partials(const double *__restrict__ part, int n)
 {
   double a = 0.0;
-  for (int i = threadIdx.x; i < n; i += kRT) a += part[i];
-  return bsum(a);
+#pragma unroll 8
+  for (int i = threadIdx.x; i < n; i += T) a += part[i];
+  return bsum<T>(a);
 }
 
 // The inner solve's scalars.  rr[i & 1] is |r|^2 at iteration i (two, so that
 // the workgroups of k_cg_ep can read the old one while the new one is
-// written); iteration i and later do nothing once done_at <= i.
+// written), alpha[i & 1] its step; iteration i and later do nothing once
+// done_at <= i, nor the rest of an iteration that breaks off once hop_at <= i.
 struct CgScal {
-  double rr[2], stop, alpha;
-  uint32_t done_at, iters, broke, pad;
+  double rr[2], alpha[2], stop;
+  uint32_t done_at, hop_at, iters, broke;
 };
 
 // What the host learns after every iteration that ran, in one word of its own
@@ -132,8 +141,8 @@ __global__ void __launch_bounds__(kRT) k_cg_begin(CgScal *__restrict__ s, const 
   if (threadIdx.x == 0) {
     s->rr[0] = rr;
     s->stop = rel_tol * rel_tol * rr;
-    s->alpha = 0.0;
-    s->done_at = 0xffffffffu;
+    s->alpha[0] = s->alpha[1] = 0.0;
+    s->done_at = s->hop_at = 0xffffffffu;
     s->iters = s->broke = 0;
   }
 }
@@ -149,77 +158,77 @@ __global__ void __launch_bounds__(kRT) k_cg_fold(const CgScal *__restrict__ s, u
   if (threadIdx.x == 0) out[blockIdx.x] = a;
 }
 
-// r -= a Ap, partial |r|^2.   (r: precision PE; Ap: PP)
-template <int PE, int PP>
-__global__ void __launch_bounds__(kRT) k_cg_r(CgScal *__restrict__ s, uint32_t it, const double *__restrict__ tt, int ntt,
-                                              const void *__restrict__ Ap, void *__restrict__ r, uint64_t npts, uint32_t M,
-                                              double *__restrict__ partial)
+// a = |r|^2 / |t|^2 from the partial sums of |t|^2, by one workgroup.  |t|^2 not
+// positive (the accuracy floor): iteration `it` ends without an update.
+__global__ void __launch_bounds__(kAT) k_cg_alpha(CgScal *__restrict__ s, uint32_t it, const double *__restrict__ tt, int n)
 {
-  typedef typename Pt<PE>::A A;
   if (s->done_at <= it) return;
-  const double pap = sum_partials(tt, ntt);
-  const bool ok = pap > 0.0;
-  const double a = ok ? s->rr[it & 1] / pap : 0.0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    s->alpha = a;
-    s->broke = ok ? 0u : 1u;
-  }
-  if (!ok) return;
-  double acc = 0.0;
-  for (uint64_t t = blockIdx.x * (uint64_t)kRT + threadIdx.x; t < npts; t += (uint64_t)gridDim.x * kRT) {
-    const uint64_t q = t / M;
-    const uint32_t m = (uint32_t)(t % M);
-    A apv[24], rv[24];
-    load_pt<PP, A>(Ap, q, M, m, apv);
-    load_pt<PE, A>(r, q, M, m, rv);
-#pragma unroll
-    for (int j = 0; j < 24; j++) {
-      rv[j] -= (A)a * apv[j];
-      acc += (double)rv[j] * (double)rv[j];
+  const double pap = sum_partials<kAT>(tt, n);
+  if (threadIdx.x == 0) {
+    const bool ok = pap > 0.0;
+    s->alpha[it & 1] = ok ? s->rr[it & 1] / pap : 0.0;
+    if (!ok) {
+      s->broke = 1u;
+      s->hop_at = it;
     }
-    store_pt<PE, A>(r, q, M, m, rv);
   }
-  acc = bsum(acc);
-  if (threadIdx.x == 0) partial[blockIdx.x] = acc;
 }
 
-// e += a p (first: e = a p), p = r + b p, and the iteration's outcome.
-template <int PE, int PP>
+// p' = r + b p and the iteration's outcome; e is brought up to date every other
+// iteration and at the end: PAIR: e += a' q + a p with q, a' the last
+// iteration's p and a, and p' goes over q.  Otherwise p' goes to another field,
+// p and a are left to the next iteration, or if it is the last: e += a p and
+// no p'.  first: e = ... instead of e += ...
+template <int PE, int PP, bool PAIR>
 __global__ void __launch_bounds__(kRT) k_cg_ep(CgScal *__restrict__ s, uint32_t it, const double *__restrict__ rpart, int nr,
-                                               const void *__restrict__ r, void *__restrict__ p, void *__restrict__ e,
-                                               uint64_t npts, uint32_t M, int first, uint64_t *word)
+                                               const void *__restrict__ r, const void *__restrict__ p, void *pn,
+                                               void *__restrict__ e, uint64_t npts, uint32_t M, int first, int last,
+                                               uint64_t *word)
 {
   typedef typename Pt<PE>::A A;
   if (s->done_at <= it) return;
-  if (s->broke) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      s->done_at = it + 1;
-      tell_host(word, it + 1, true, true);
-    }
-    return;
+  const bool broke = s->broke != 0;
+  double rr_new = 0.0, b = 0.0;
+  bool done = true;
+  if (!broke) {
+    rr_new = sum_partials<kRT>(rpart, nr);
+    b = rr_new / s->rr[it & 1];
+    done = !(rr_new > s->stop);
   }
-  const double rr_new = sum_partials(rpart, nr), b = rr_new / s->rr[it & 1], a = s->alpha;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    const bool done = !(rr_new > s->stop);
-    s->rr[(it + 1) & 1] = rr_new;
-    s->iters = it + 1;
-    if (done) s->done_at = it + 1;
-    tell_host(word, it + 1, done, false);
+    if (!broke) {
+      s->rr[(it + 1) & 1] = rr_new;
+      s->iters = it + 1;
+    }
+    if (done) s->done_at = s->hop_at = it + 1;
+    tell_host(word, it + 1, done, broke);
   }
+  const bool end = done || last;
+  if (broke && !PAIR) return;
+  const A a = broke ? (A)0 : (A)s->alpha[it & 1], a1 = PAIR ? (A)s->alpha[(it + 1) & 1] : (A)0;
   for (uint64_t t = blockIdx.x * (uint64_t)kRT + threadIdx.x; t < npts; t += (uint64_t)gridDim.x * kRT) {
     const uint64_t q = t / M;
     const uint32_t m = (uint32_t)(t % M);
-    A rv[24], pv[24], ev[24];
-    load_pt<PE, A>(r, q, M, m, rv);
+    A pv[24], v[24];
     load_pt<PP, A>(p, q, M, m, pv);
-    if (!first) load_pt<PE, A>(e, q, M, m, ev);
+    if (PAIR || end) {
+      A ev[24];
+      if (!first) load_pt<PE, A>(e, q, M, m, ev);
+      if (PAIR) load_pt<PP, A>(pn, q, M, m, v);
 #pragma unroll
-    for (int j = 0; j < 24; j++) {
-      ev[j] = (first ? (A)0 : ev[j]) + (A)a * pv[j];
-      pv[j] = rv[j] + (A)b * pv[j];
+      for (int j = 0; j < 24; j++) {
+        ev[j] = first ? (A)0 : ev[j];
+        if (PAIR) ev[j] += a1 * v[j];
+        if (!broke) ev[j] += a * pv[j];
+      }
+      store_pt<PE, A>(e, q, M, m, ev);
     }
-    store_pt<PE, A>(e, q, M, m, ev);
-    store_pt<PP, A>(p, q, M, m, pv);
+    if (!end) {
+      load_pt<PE, A>(r, q, M, m, v);
+#pragma unroll
+      for (int j = 0; j < 24; j++) v[j] += (A)b * pv[j];
+      store_pt<PP, A>(pn, q, M, m, v);
+    }
   }
 }
 
@@ -267,19 +276,42 @@ __global__ void __launch_bounds__(kRT) k_final(const double *__restrict__ partia
   if (threadIdx.x == 0) out[0] = a;
 }
 
-// Pinned host memory of a thread's solves, kept until the process ends: the
-// word the device reports iterations in, and a sum.
+// Pinned host memory of a solve: the word the device reports iterations in, and
+// a sum.  A solve takes one for itself and gives it back; up to kWords unused
+// ones are kept for later solves.
 struct HostWords {
   uint64_t word;
   double sum;
 };
 
-int host_words(HostWords **w)
+constexpr size_t kWords = 8;
+std::mutex g_words_mu;
+std::vector<HostWords *> g_words;
+
+int take_words(HostWords **w)
 {
-  static thread_local HostWords *g = nullptr;
-  if (!g) GBX_HIP(hipHostMalloc(&g, sizeof(HostWords), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
-  *w = g;
+  {
+    std::lock_guard<std::mutex> lk(g_words_mu);
+    if (!g_words.empty()) {
+      *w = g_words.back();
+      g_words.pop_back();
+      return GBX_OK;
+    }
+  }
+  GBX_HIP(hipHostMalloc(w, sizeof(HostWords), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
   return GBX_OK;
+}
+
+void give_words(HostWords *w)
+{
+  {
+    std::lock_guard<std::mutex> lk(g_words_mu);
+    if (g_words.size() < kWords) {
+      g_words.push_back(w);
+      return;
+    }
+  }
+  (void)hipHostFree(w);
 }
 
 // Device memory of one solve: its fields and scalars in one allocation (eight
@@ -290,11 +322,14 @@ struct Workspace {
   hipStream_t st = nullptr;
   std::vector<gbx_spinor_s *> fields;
   std::vector<size_t> at;
+  HostWords *words = nullptr;
   ~Workspace()
   {
-    if (!base) return;
-    (void)hipStreamSynchronize(st);
-    (void)hipFree(base);
+    if (base) {
+      (void)hipStreamSynchronize(st);
+      (void)hipFree(base);
+    }
+    if (words) give_words(words);  // no kernel writes to them any more
   }
   size_t take(size_t n)
   {
@@ -341,13 +376,15 @@ struct Scratch {
     tt_at = w.take(sizeof(double) * ntt);
     fold_at = w.take(sizeof(double) * kFold);
   }
-  int init(const Workspace &w)
+  int init(Workspace &w)
   {
     scal = (CgScal *)(w.base + scal_at);
     partial = (double *)(w.base + part_at);
     tt = (double *)(w.base + tt_at);
     fold = (double *)(w.base + fold_at);
-    return host_words(&host);
+    GBX_TRY(take_words(&w.words));
+    host = w.words;
+    return GBX_OK;
   }
   // The sum of n partial sums on the host (waits for the stream).
   int fetch(hipStream_t st, int n, double *v)
@@ -394,18 +431,25 @@ struct NormalOp {
   }
 };
 
-// An application inside the inner CG: it does nothing once *skip <= skip_at,
-// and puts the partial sums of |t|^2, t = M x, into tt.
+// An application inside the inner CG: it does nothing once *skip <= skip_at, and
+// its last kernel sums into `partial`: of M, |out|^2; of M^dag, |r|^2 after
+// r -= *a out in place of writing out.
 struct Step {
   const uint32_t *skip = nullptr;
   uint32_t skip_at = 0;
-  double *tt = nullptr;
+  double *partial = nullptr;
+  gbx_spinor_s *r = nullptr;
+  const double *a = nullptr;
   dhop_fuse fuse(bool sum) const
   {
     dhop_fuse f;
     f.skip = skip;
     f.skip_at = skip_at;
-    f.partial = sum ? tt : nullptr;
+    if (sum) {
+      f.partial = partial;
+      f.resid = r;
+      f.resid_a = a;
+    }
     return f;
   }
 };
@@ -447,27 +491,29 @@ int mooee_plus_dhop(const gbx_gauge_s *u, const dhop_cfg &cfg, gbx_spinor_s *out
 int apply_schur(const NormalOp &op, gbx_spinor_s *y, const gbx_spinor_s *x, int dag, hipStream_t st,
                 const Step &step = Step())
 {
-  const bool sum = step.tt && !dag;
   if (op.kind == OP_DWF) {
     GBX_TRY(mooee_inv_dhop(op.uo, op.co, op.to, x, &op.dwf, dag, st, step.fuse(false)));
-    return mooee_plus_dhop(op.ue, op.ce, y, x, op.to, &op.dwf, dag, -0.25, st, step.fuse(sum));
+    return mooee_plus_dhop(op.ue, op.ce, y, x, op.to, &op.dwf, dag, -0.25, st, step.fuse(true));
   }
   GBX_TRY(hop(op.uo, op.co, op.to, x, dag, 0.0, 1.0, nullptr, st, step.fuse(false)));
-  return hop(op.ue, op.ce, y, op.to, dag, 1.0, -op.kappa * op.kappa, x, st, step.fuse(sum));
+  return hop(op.ue, op.ce, y, op.to, dag, 1.0, -op.kappa * op.kappa, x, st, step.fuse(true));
 }
 
-// y = A x.  Whole lattice: t = x - kappa Dhop x; y = t - kappa Dhop^dag t.
-int apply_normal(const NormalOp &op, gbx_spinor_s *y, const gbx_spinor_s *x, hipStream_t st, const Step &step = Step())
+// y = M x or M^dag x on the whole lattice, x - kappa Dhop x.
+int apply_m(const NormalOp &op, gbx_spinor_s *y, const gbx_spinor_s *x, int dag, hipStream_t st, const Step &step = Step())
 {
-  if (op.eo) {
-    GBX_TRY(apply_schur(op, op.t, x, 0, st, step));
-    return apply_schur(op, y, op.t, 1, st, step);
-  }
-  GBX_TRY(hop(op.ue, op.ce, op.t, x, 0, 1.0, -op.kappa, x, st, step.fuse(step.tt != nullptr)));
-  return hop(op.ue, op.ce, y, op.t, 1, 1.0, -op.kappa, op.t, st, step.fuse(false));
+  if (op.eo) return apply_schur(op, y, x, dag, st, step);
+  return hop(op.ue, op.ce, y, x, dag, 1.0, -op.kappa, x, st, step.fuse(true));
 }
 
-// Partial sums of |t|^2 an application leaves in Step::tt.
+// y = A x by way of t.
+int apply_normal(const NormalOp &op, gbx_spinor_s *y, const gbx_spinor_s *x, hipStream_t st)
+{
+  GBX_TRY(apply_m(op, op.t, x, 0, st));
+  return apply_m(op, y, op.t, 1, st);
+}
+
+// Partial sums an application leaves in Step::partial.
 uint32_t normal_partials(const NormalOp &op) { return dhop_workgroups(op.ue, op.t, op.ce); }
 
 // Waits until the device has reported iteration `seen` + 1 of the inner solve.
@@ -490,39 +536,54 @@ int next_word(const HostWords *h, uint32_t seen, hipStream_t st, uint64_t *word)
   }
 }
 
-// Inner CG on A e = scale * src (src FP64): e, r in precision PE; p, Ap and
-// the operator's temporaries in PP (the gauge field's).  *it_out iterations
-// ran; e is not written if that is 0.
+// Inner CG on A e = scale * src (src FP64): e, r in precision PE; p, its other
+// buffer p2 and the operator's temporaries in PP (the gauge field's).  *it_out
+// iterations ran; e is not written if that is 0.
 template <int PE, int PP>
-int inner_cg(const NormalOp &op, gbx_spinor_s *e, gbx_spinor_s *r, gbx_spinor_s *p, gbx_spinor_s *Ap, const gbx_spinor_s *src,
+int inner_cg(const NormalOp &op, gbx_spinor_s *e, gbx_spinor_s *r, gbx_spinor_s *p, gbx_spinor_s *p2, const gbx_spinor_s *src,
              double scale, double rel_tol, int max_iter, uint32_t *it_out, int *applies, Scratch &sc, hipStream_t st)
 {
   constexpr uint32_t kAhead = 3;  // iterations enqueued beyond the last one reported
   const uint64_t npts = r->geom->vol * (uint64_t)r->M;
   const int nb = blocks_for(npts);
-  const int ntt = (int)normal_partials(op);
+  const int np = (int)normal_partials(op);
   const dim3 grid((unsigned)nb), block(kRT);
   HostWords *h = sc.host;
   __atomic_store_n(&h->word, 0ull, __ATOMIC_RELEASE);
   hipLaunchKernelGGL((k_cg_start<PE, PP>), grid, block, 0, st, scale, src->d, r->d, p->d, npts, r->M, sc.partial);
   hipLaunchKernelGGL(k_cg_begin, dim3(1), block, 0, st, sc.scal, (const double *)sc.partial, nb, rel_tol);
   GBX_HIP(hipGetLastError());
+  auto fold = [&](uint32_t it, const double *part, int *n) -> const double * {
+    if (*n <= kPlain) return part;
+    hipLaunchKernelGGL(k_cg_fold, dim3(kFold), block, 0, st, (const CgScal *)sc.scal, it, part, *n, sc.fold);
+    *n = kFold;
+    return sc.fold;
+  };
+  gbx_spinor_s *pp[2] = {p, p2};
   auto enqueue = [&](uint32_t it) -> int {
+    gbx_spinor_s *pi = pp[it & 1], *pn = pp[~it & 1];
     Step step;
     step.skip = &sc.scal->done_at;
     step.skip_at = it;
-    step.tt = sc.tt;
-    GBX_TRY(apply_normal(op, Ap, p, st, step));
-    const double *tt = sc.tt;
-    int n = ntt;
-    if (ntt > kPlain) {
-      hipLaunchKernelGGL(k_cg_fold, dim3(kFold), block, 0, st, (const CgScal *)sc.scal, it, tt, ntt, sc.fold);
-      tt = sc.fold;
-      n = kFold;
-    }
-    hipLaunchKernelGGL((k_cg_r<PE, PP>), grid, block, 0, st, sc.scal, it, tt, n, Ap->d, r->d, npts, r->M, sc.partial);
-    hipLaunchKernelGGL((k_cg_ep<PE, PP>), grid, block, 0, st, sc.scal, it, (const double *)sc.partial, nb, r->d, p->d, e->d,
-                       npts, r->M, it == 0 ? 1 : 0, &h->word);
+    step.partial = sc.tt;
+    GBX_TRY(apply_m(op, op.t, pi, 0, st, step));
+    int n = np;
+    const double *tt = fold(it, sc.tt, &n);
+    hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(kAT), 0, st, sc.scal, it, tt, n);
+    step.skip = &sc.scal->hop_at;
+    step.partial = sc.tt;
+    step.r = r;
+    step.a = &sc.scal->alpha[it & 1];
+    GBX_TRY(apply_m(op, pn, op.t, 1, st, step));  // pn: not written
+    n = np;
+    const double *rp = fold(it, sc.tt, &n);
+    const int first = it < 2, last = it + 1 == (uint32_t)max_iter;
+    if (it & 1)
+      hipLaunchKernelGGL((k_cg_ep<PE, PP, true>), grid, block, 0, st, sc.scal, it, rp, n, r->d, pi->d, pn->d, e->d, npts, r->M,
+                         first, last, &h->word);
+    else
+      hipLaunchKernelGGL((k_cg_ep<PE, PP, false>), grid, block, 0, st, sc.scal, it, rp, n, r->d, pi->d, pn->d, e->d, npts, r->M,
+                         first, last, &h->word);
     GBX_HIP(hipGetLastError());
     return GBX_OK;
   };
@@ -541,15 +602,15 @@ int inner_cg(const NormalOp &op, gbx_spinor_s *e, gbx_spinor_s *r, gbx_spinor_s 
   return GBX_OK;
 }
 
-int inner_dispatch(const NormalOp &op, gbx_spinor_s *e, gbx_spinor_s *r, gbx_spinor_s *p, gbx_spinor_s *Ap,
+int inner_dispatch(const NormalOp &op, gbx_spinor_s *e, gbx_spinor_s *r, gbx_spinor_s *p, gbx_spinor_s *p2,
                    const gbx_spinor_s *src, double scale, double tol, int maxit, uint32_t *it, int *applies, Scratch &sc,
                    hipStream_t st)
 {
-  if (e->prec == GBX_F64) return inner_cg<GBX_F64, GBX_F64>(op, e, r, p, Ap, src, scale, tol, maxit, it, applies, sc, st);
+  if (e->prec == GBX_F64) return inner_cg<GBX_F64, GBX_F64>(op, e, r, p, p2, src, scale, tol, maxit, it, applies, sc, st);
   switch (p->prec) {
-  case GBX_F32: return inner_cg<GBX_F32, GBX_F32>(op, e, r, p, Ap, src, scale, tol, maxit, it, applies, sc, st);
-  case GBX_F16: return inner_cg<GBX_F32, GBX_F16>(op, e, r, p, Ap, src, scale, tol, maxit, it, applies, sc, st);
-  default: return inner_cg<GBX_F32, GBX_BF16>(op, e, r, p, Ap, src, scale, tol, maxit, it, applies, sc, st);
+  case GBX_F32: return inner_cg<GBX_F32, GBX_F32>(op, e, r, p, p2, src, scale, tol, maxit, it, applies, sc, st);
+  case GBX_F16: return inner_cg<GBX_F32, GBX_F16>(op, e, r, p, p2, src, scale, tol, maxit, it, applies, sc, st);
+  default: return inner_cg<GBX_F32, GBX_BF16>(op, e, r, p, p2, src, scale, tol, maxit, it, applies, sc, st);
   }
 }
 
@@ -620,10 +681,10 @@ int solve(const gbx_gauge_s *u_hi, const gbx_gauge_s *u_lo, gbx_spinor_s *x, con
   const int plo = u_lo ? u_lo->prec : GBX_F64;
   const int pe = u_lo ? GBX_F32 : GBX_F64;
   Workspace w;
-  gbx_spinor_s r, t, y, e, ri, p, Ap, tl;
+  gbx_spinor_s r, t, y, e, ri, p, p2, tl;
   for (gbx_spinor_s *f : {&r, &t, &y}) w.field(*f, g, Ls, GBX_F64, b->basis);
   for (gbx_spinor_s *f : {&e, &ri}) w.field(*f, g, Ls, pe, b->basis);
-  for (gbx_spinor_s *f : {&p, &Ap, &tl}) w.field(*f, g, Ls, plo, b->basis);
+  for (gbx_spinor_s *f : {&p, &p2, &tl}) w.field(*f, g, Ls, plo, b->basis);
   NormalOp op_hi{false, u_hi, nullptr, prm->kappa, &t, nullptr};
   NormalOp op_lo{false, u_lo ? u_lo : u_hi, nullptr, prm->kappa, &tl, nullptr};
   op_hi.shapes();
@@ -648,7 +709,7 @@ int solve(const gbx_gauge_s *u_hi, const gbx_gauge_s *u_lo, gbx_spinor_s *x, con
     if (rel <= prm->tol || st.outer_iters >= prm->max_outer || !(rr > 0.0)) break;
     const double scale = std::sqrt(N) / std::sqrt(rr);
     uint32_t it = 0;
-    GBX_TRY(inner_dispatch(op_lo, &e, &ri, &p, &Ap, &r, scale, prm->inner_tol, prm->max_inner, &it, &st.lo_applies, sc, s));
+    GBX_TRY(inner_dispatch(op_lo, &e, &ri, &p, &p2, &r, scale, prm->inner_tol, prm->max_inner, &it, &st.lo_applies, sc, s));
     if (it) GBX_TRY(axpy_into_f64(1.0 / scale, &e, x, s));
     st.inner_iters += (int)it;
     st.outer_iters++;
@@ -710,11 +771,11 @@ int solve_schur(int kind, const gbx_dwf_params *dwf, const gbx_gauge_s *const u_
   const int plo = u_lo ? u_lo[0]->prec : GBX_F64;
   const int pe = u_lo ? GBX_F32 : GBX_F64;
   Workspace w;
-  gbx_spinor_s bp, r, y, t, to, e, ri, p, Ap, tl, tol_, ro;
+  gbx_spinor_s bp, r, y, t, to, e, ri, p, p2, tl, tol_, ro;
   for (gbx_spinor_s *f : {&bp, &r, &y, &t}) w.field(*f, g, Ls, GBX_F64, basis);
   for (gbx_spinor_s *f : {&to, &ro}) w.field(*f, g1, Ls, GBX_F64, basis);
   for (gbx_spinor_s *f : {&e, &ri}) w.field(*f, g, Ls, pe, basis);
-  for (gbx_spinor_s *f : {&p, &Ap, &tl}) w.field(*f, g, Ls, plo, basis);
+  for (gbx_spinor_s *f : {&p, &p2, &tl}) w.field(*f, g, Ls, plo, basis);
   w.field(tol_, g1, Ls, plo, basis);
   NormalOp op_hi{true, u_hi[0], u_hi[1], kappa, &t, &to};
   NormalOp op_lo{true, u_lo ? u_lo[0] : u_hi[0], u_lo ? u_lo[1] : u_hi[1], kappa, &tl, &tol_};
@@ -755,7 +816,7 @@ int solve_schur(int kind, const gbx_dwf_params *dwf, const gbx_gauge_s *const u_
     if (!(yy > 0.0)) break;
     const double scale = std::sqrt(N) / std::sqrt(yy);
     uint32_t it = 0;
-    GBX_TRY(inner_dispatch(op_lo, &e, &ri, &p, &Ap, &y, scale, prm->inner_tol, prm->max_inner, &it, &st.lo_applies, sc, s));
+    GBX_TRY(inner_dispatch(op_lo, &e, &ri, &p, &p2, &y, scale, prm->inner_tol, prm->max_inner, &it, &st.lo_applies, sc, s));
     if (it) GBX_TRY(axpy_into_f64(1.0 / scale, &e, x[0], s));
     st.inner_iters += (int)it;
     st.outer_iters++;

@@ -231,7 +231,7 @@ int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in,
   GBX_TRY(dhop_cfg_check(c, u, in));
   const int s5 = fuse ? fuse->s5 : (int)dhop_fuse::NONE;
   const bool axpby = s5 == dhop_fuse::MOOEE || (s5 == dhop_fuse::NONE && !(alpha == 0.0 && beta == 1.0));
-  const bool red = fuse && fuse->partial;
+  const int red = !fuse || !fuse->partial ? RED_NONE : dag ? RED_RESID : RED_OUT;
   GBX_CHECK(!exact || ((u->prec == GBX_F64 || u->prec == GBX_F32) && !u->comp12 && !axpby), GBX_EUNSUPPORTED,
             "dhop: the reference-rounding kernel takes FP64 / FP32 fields with 18-real links");
   const bool td = in->basis == GBX_BASIS_TDIAG;
@@ -290,10 +290,18 @@ int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in,
     a.skip = fuse->skip;
     a.skip_at = fuse->skip_at;
     a.partial = fuse->partial;
+    if (red == RED_RESID) {
+      const gbx_spinor_s *r = fuse->resid;
+      GBX_CHECK(axpby && r && r->d && fuse->resid_a && r->geom == out->geom && r->M == in->M &&
+                    r->prec == (in->prec == GBX_F64 ? GBX_F64 : GBX_F32) && r->d != in->d && r->d != center->d,
+                GBX_EINVAL, "dhop: no such residual update");
+      a.r = r->d;
+      a.a = fuse->resid_a;
+    }
   }
   if (s5 != dhop_fuse::NONE || red) {
     a.lds = std::min(a.lds, (size_t)160 * 1024 - 128);  // a residency pad leaves room for the sum's scratch
-    GBX_CHECK(whole && !exact && !c.projected_ghosts && (!red || (axpby && !dag)) && (s5 == dhop_fuse::NONE || !td),
+    GBX_CHECK(whole && !exact && !c.projected_ghosts && (!red || axpby) && (s5 == dhop_fuse::NONE || !td),
               GBX_EUNSUPPORTED, "dhop: no such fused form");
     int epi = EPI_AXPBY;
     if (s5 != dhop_fuse::NONE) {

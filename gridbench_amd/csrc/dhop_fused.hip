@@ -16,40 +16,50 @@ namespace dhopk {
 
 namespace {
 
-template <int P, bool DAG, bool C12, int EPI, bool TD, bool RED>
+template <int P, bool DAG, bool C12, int EPI, bool TD, int RED>
 void pick_pf(int pf, const LaunchArgs &a)
 {
   if (pf) launch_t<P, DAG, C12, EPI, 1, false, false, TD, RED>(a);
   else launch_t<P, DAG, C12, EPI, 0, false, false, TD, RED>(a);
 }
 
+template <int P, bool C12, int EPI, bool TD = false>
+void pick_red(bool dag, int red, int pf, const LaunchArgs &a)
+{
+  if (dag) {
+    if (red) pick_pf<P, true, C12, EPI, TD, RED_RESID>(pf, a);
+    else pick_pf<P, true, C12, EPI, TD, RED_NONE>(pf, a);
+  } else {
+    if (red) pick_pf<P, false, C12, EPI, TD, RED_OUT>(pf, a);
+    else pick_pf<P, false, C12, EPI, TD, RED_NONE>(pf, a);
+  }
+}
+
 template <int P, bool C12>
-void pick_epi(int epi, bool dag, bool td, bool red, int pf, const LaunchArgs &a)
+void pick_epi(int epi, bool dag, bool td, int red, int pf, const LaunchArgs &a)
 {
   if (epi == EPI_S5INV) {
-    if (dag) pick_pf<P, true, C12, EPI_S5INV, false, false>(pf, a);
-    else pick_pf<P, false, C12, EPI_S5INV, false, false>(pf, a);
+    if (dag) pick_pf<P, true, C12, EPI_S5INV, false, RED_NONE>(pf, a);
+    else pick_pf<P, false, C12, EPI_S5INV, false, RED_NONE>(pf, a);
   } else if (epi == EPI_S5) {
-    if (dag) pick_pf<P, true, C12, EPI_S5, false, false>(pf, a);
-    else if (red) pick_pf<P, false, C12, EPI_S5, false, true>(pf, a);
-    else pick_pf<P, false, C12, EPI_S5, false, false>(pf, a);
+    pick_red<P, C12, EPI_S5>(dag, red, pf, a);
   } else if (epi == EPI_S5X) {
-    if (dag) pick_pf<P, true, C12, EPI_S5X, false, false>(pf, a);
-    else if (red) pick_pf<P, false, C12, EPI_S5X, false, true>(pf, a);
-    else pick_pf<P, false, C12, EPI_S5X, false, false>(pf, a);
+    pick_red<P, C12, EPI_S5X>(dag, red, pf, a);
   } else {
     if constexpr (P == GBX_F64 || P == GBX_F32) {
       if (td) {
-        pick_pf<P, false, C12, EPI_AXPBY, true, true>(pf, a);
+        if (dag) pick_pf<P, true, C12, EPI_AXPBY, true, RED_RESID>(pf, a);
+        else pick_pf<P, false, C12, EPI_AXPBY, true, RED_OUT>(pf, a);
         return;
       }
     }
-    pick_pf<P, false, C12, EPI_AXPBY, false, true>(pf, a);
+    if (dag) pick_pf<P, true, C12, EPI_AXPBY, false, RED_RESID>(pf, a);
+    else pick_pf<P, false, C12, EPI_AXPBY, false, RED_OUT>(pf, a);
   }
 }
 
 template <int P>
-void pick_c12(int epi, bool dag, bool c12, bool td, bool red, int pf, const LaunchArgs &a)
+void pick_c12(int epi, bool dag, bool c12, bool td, int red, int pf, const LaunchArgs &a)
 {
   if (c12) pick_epi<P, true>(epi, dag, td, red, pf, a);
   else pick_epi<P, false>(epi, dag, td, red, pf, a);
@@ -57,7 +67,7 @@ void pick_c12(int epi, bool dag, bool c12, bool td, bool red, int pf, const Laun
 
 }  // namespace
 
-void launch_fused(int prec, int epi, bool dag, bool c12, bool td, bool red, int pf, const LaunchArgs &a)
+void launch_fused(int prec, int epi, bool dag, bool c12, bool td, int red, int pf, const LaunchArgs &a)
 {
   switch (prec) {
   case GBX_F64: pick_c12<GBX_F64>(epi, dag, c12, td, red, pf, a); break;

@@ -18,19 +18,71 @@ enum {
   EPI_S5X = 4     // EPI_S5 in workgroups that hold whole columns of slices
 };
 
+// What it sums.
+enum {
+  RED_NONE = 0,
+  RED_OUT = 1,   // |out|^2
+  RED_RESID = 2  // r -= *a out in place of storing out, |r|^2
+};
+
 template <typename A> struct Epi {
   A alpha, beta;
   A d, mass;             // domain-wall terms: d = 5 - M5
   uint32_t Ls;
   const uint32_t *skip;  // nothing runs if *skip <= skip_at
   uint32_t skip_at;
-  double *partial;       // RED: |out|^2 of every workgroup
+  double *partial;       // the sum of every workgroup
+  void *r;               // RED_RESID: a field of the arithmetic type
+  const double *a;
 };
+
+// The residual's reals of chunks k0 .. k0+G-1 of a point (RED_RESID).
+template <int P, int RED, int G>
+__device__ __forceinline__ void load_resid(uint32_t q, uint32_t M, uint32_t m, int k0,
+                                           const Epi<typename dev::Traits<P>::acc> &e, typename dev::Traits<P>::acc *x)
+{
+  typedef typename dev::Traits<P>::acc A;
+  if constexpr (RED == RED_RESID) {
+    constexpr int PR = P == GBX_F64 ? GBX_F64 : GBX_F32, RR = dev::Traits<PR>::R, RC = dev::Traits<PR>::NCH;
+    constexpr int N = dev::Traits<P>::R / RR;
+#pragma unroll
+    for (int i = 0; i < G * N; i++) dev::load_chunk<PR, A>(e.r, ((uint64_t)q * RC + k0 * N + i) * M + m, x + i * RR);
+  }
+}
+
+// The end of an epilogue for chunk k of a point: store it, or update the
+// residual's reals x by it.
+template <int P, int RED>
+__device__ __forceinline__ void finish_chunk(void *__restrict__ out, uint32_t q, uint32_t M, uint32_t m, int k,
+                                             const Epi<typename dev::Traits<P>::acc> &e, typename dev::Traits<P>::acc a,
+                                             const typename dev::Traits<P>::acc *v, typename dev::Traits<P>::acc *x, bool nt,
+                                             double &norm)
+{
+  typedef typename dev::Traits<P>::acc A;
+  constexpr int NCH = dev::Traits<P>::NCH, R = dev::Traits<P>::R;
+  if constexpr (RED == RED_RESID) {
+    constexpr int PR = P == GBX_F64 ? GBX_F64 : GBX_F32, RR = dev::Traits<PR>::R, RC = dev::Traits<PR>::NCH, N = R / RR;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      x[j] -= a * v[j];
+      norm += (double)x[j] * (double)x[j];
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++)
+      dev::store_chunk<PR, A>(e.r, ((uint64_t)q * RC + k * N + i) * M + m, x + i * RR, false);
+  } else {
+    if constexpr (RED == RED_OUT) {
+#pragma unroll
+      for (int j = 0; j < R; j++) norm += (double)v[j] * (double)v[j];
+    }
+    dev::store_chunk<P, A>(out, ((uint64_t)q * NCH + k) * M + m, v, nt);
+  }
+}
 
 // out = Mooee c + beta r for one (site, minor) point: the neighbour slice each
 // chirality hops from (up in s for P-, down for P+, exchanged for DAG) is read
 // from memory next to the point's own, mostly the same cache lines.
-template <int P, bool DAG, bool RED>
+template <int P, bool DAG, int RED>
 __device__ __forceinline__ void store_s5(void *__restrict__ out, const void *__restrict__ c, uint32_t q, uint32_t M, uint32_t m,
                                          const Epi<typename dev::Traits<P>::acc> &e, typename dev::Traits<P>::acc *rr,
                                          typename dev::Traits<P>::acc *ri, bool nt, double &norm)
@@ -42,23 +94,24 @@ __device__ __forceinline__ void store_s5(void *__restrict__ out, const void *__r
   const uint32_t s = m % e.Ls;
   const uint32_t mdn = s == 0 ? m + e.Ls - 1 : m - 1, mup = s == e.Ls - 1 ? m - (e.Ls - 1) : m + 1;
   const A cdn = s == 0 ? e.mass : (A)-1, cup = s == e.Ls - 1 ? e.mass : (A)-1;
+  const A a = RED == RED_RESID ? (A)*e.a : (A)0;
 #pragma unroll
   for (int k = 0; k < NCH; k++) {
     if (R == 8) __builtin_amdgcn_sched_barrier(0);  // one 16-bit chunk at a time: 3 or 4 loads of 8 reals
-    A own[R], dn[R], up[R], v[R];
+    A own[R], dn[R], up[R], v[R], x[R];
     const bool has_dn = DAG ? (k + 1) * R > 12 : k * R < 12, has_up = DAG ? k * R < 12 : (k + 1) * R > 12;
     dev::load_chunk<P, A>(c, base + (uint64_t)k * M + m, own);
     if (has_dn) dev::load_chunk<P, A>(c, base + (uint64_t)k * M + mdn, dn);
     if (has_up) dev::load_chunk<P, A>(c, base + (uint64_t)k * M + mup, up);
+    load_resid<P, RED, 1>(q, M, m, k, e, x);
 #pragma unroll
     for (int j = 0; j < R; j++) {
       const int r = k * R + j;
       const bool down = (r < 12) != DAG;
       const A acc = e.d * own[j] + (down ? cdn : cup) * (down ? dn[j] : up[j]);
       v[j] = acc + e.beta * ((r & 1) ? ri[r >> 1] : rr[r >> 1]);
-      if (RED) norm += (double)v[j] * (double)v[j];
     }
-    dev::store_chunk<P, A>(out, base + (uint64_t)k * M + m, v, nt);
+    finish_chunk<P, RED>(out, q, M, m, k, e, a, v, x, nt, norm);
   }
 }
 
@@ -67,12 +120,11 @@ __device__ __forceinline__ void store_s5(void *__restrict__ out, const void *__r
 // and takes the neighbour slices from LDS, a chirality at a time (16-bit
 // fields all three chunks at once).  Half the loads of store_s5 and fewer
 // registers (FP32 72 instead of 81, 73 instead of 96 with the norm: 7 or 6
-// wavefronts a SIMD instead of 5).  What bounds the kernel is still the legs' gathers: 24^4 x
-// Ls16 FP64 869 -> 863 us, the domain-wall solve at 16^4 x Ls12, FP32 inner,
-// 16.40 -> 16.28 ms.  Every thread calls it; `w` is the point's index in the
-// workgroup, s its slice, `active`
-// whether it has one.
-template <int P, bool DAG, bool RED>
+// wavefronts a SIMD instead of 5).  What bounds the kernel is still the legs'
+// gathers: 24^4 x Ls16 FP64 869 -> 863 us, the domain-wall solve at 16^4 x
+// Ls12, FP32 inner, 16.40 -> 16.28 ms.  Every thread calls it; `w` is the
+// point's index in the workgroup, s its slice, `active` whether it has one.
+template <int P, bool DAG, int RED>
 __device__ __forceinline__ void store_s5x(void *__restrict__ out, const void *__restrict__ c, uint32_t q, uint32_t M, uint32_t m,
                                           const Epi<typename dev::Traits<P>::acc> &e, uint32_t w, uint32_t s, bool active,
                                           unsigned char *smem, typename dev::Traits<P>::acc *rr,
@@ -86,13 +138,16 @@ __device__ __forceinline__ void store_s5x(void *__restrict__ out, const void *__
   const uint32_t th = blockDim.x;
   const uint32_t wdn = s == 0 ? w + e.Ls - 1 : w - 1, wup = s == e.Ls - 1 ? w - (e.Ls - 1) : w + 1;
   const A cdn = s == 0 ? e.mass : (A)-1, cup = s == e.Ls - 1 ? e.mass : (A)-1;
+  const A a = RED == RED_RESID ? (A)*e.a : (A)0;
 #pragma unroll
   for (int k0 = 0; k0 < NCH; k0 += G) {
     V own[G];
+    A x[G * R];
     __builtin_amdgcn_sched_barrier(0);  // c's chunks are not held across the legs
     if (active) {
 #pragma unroll
       for (int k = 0; k < G; k++) own[k] = ((const V *)c)[base + (uint64_t)(k0 + k) * M];
+      load_resid<P, RED, G>(q, M, m, k0, e, x);
     }
     __syncthreads();  // the links, or the other chirality, are no longer read
     if (active) {
@@ -116,9 +171,8 @@ __device__ __forceinline__ void store_s5x(void *__restrict__ out, const void *__
           const bool down = (r < 12) != DAG;
           const A acc = e.d * (A)own[k][j] + (down ? cdn : cup) * (A)(down ? dn[j] : up[j]);
           v[j] = acc + e.beta * ((r & 1) ? ri[r >> 1] : rr[r >> 1]);
-          if (RED) norm += (double)v[j] * (double)v[j];
         }
-        dev::store_chunk<P, A>(out, base + (uint64_t)(k0 + k) * M, v, nt);
+        finish_chunk<P, RED>(out, q, M, m, k0 + k, e, a, v, x + k * R, nt, norm);
       }
     }
   }
@@ -195,11 +249,11 @@ __device__ __forceinline__ void again(uint32_t &w, uint32_t mcc, uint32_t &sl, u
   m = w - sl * mcc;
 }
 
-// out = alpha c + beta r of one point and its |out|^2, a chunk at a time: with
+// alpha c + beta r of one point and its sum, a chunk at a time: with
 // all 24 results and their squares in registers together the 16-bit forms need
 // more than the plain kernel's 80 and lose a wavefront of six.  CG at 16^3x24
 // x Ls8, FP16 inner: 13.6 -> 13.1 ms.
-template <int P>
+template <int P, int RED>
 __device__ __forceinline__ void store_axpby_norm(void *__restrict__ out, const void *__restrict__ c, uint32_t q, uint32_t M,
                                                  uint32_t m, const Epi<typename dev::Traits<P>::acc> &e,
                                                  typename dev::Traits<P>::acc *rr, typename dev::Traits<P>::acc *ri, bool nt,
@@ -209,12 +263,15 @@ __device__ __forceinline__ void store_axpby_norm(void *__restrict__ out, const v
   typedef typename dev::Traits<P>::vec V;
   constexpr int NCH = dev::Traits<P>::NCH, R = dev::Traits<P>::R, G = NCH < 6 ? NCH : NCH / 2;
   const uint64_t base = (uint64_t)q * NCH * M + m;
+  const A a = RED == RED_RESID ? (A)*e.a : (A)0;
 #pragma unroll
   for (int k0 = 0; k0 < NCH; k0 += G) {
     V own[G];
+    A x[G * R];
     __builtin_amdgcn_sched_barrier(0);  // c's chunks are not held across the legs
 #pragma unroll
     for (int k = 0; k < G; k++) own[k] = ((const V *)c)[base + (uint64_t)(k0 + k) * M];
+    load_resid<P, RED, G>(q, M, m, k0, e, x);
 #pragma unroll
     for (int k = 0; k < G; k++) {
       __builtin_amdgcn_sched_barrier(0);
@@ -223,9 +280,8 @@ __device__ __forceinline__ void store_axpby_norm(void *__restrict__ out, const v
       for (int j = 0; j < R; j++) {
         const int r = (k0 + k) * R + j;
         v[j] = e.alpha * (A)own[k][j] + e.beta * ((r & 1) ? ri[r >> 1] : rr[r >> 1]);
-        norm += (double)v[j] * (double)v[j];
       }
-      dev::store_chunk<P, A>(out, base + (uint64_t)(k0 + k) * M, v, nt);
+      finish_chunk<P, RED>(out, q, M, m, k0 + k, e, a, v, x + k * R, nt, norm);
     }
   }
 }
@@ -249,10 +305,10 @@ __device__ __forceinline__ double block_sum(double a)
 // the lattice is swept once per minor chunk, so the 8-neighbour working set
 // is that of an mc-wide field (the links are re-read once per chunk).
 // GP: a domain part whose ghosts hold spin-projected halves from ghost0 on
-// (dhop_site_gp).  TD: fields in the GBX_BASIS_TDIAG spin basis.  RED: also
-// |out|^2 of the workgroup's values (before their rounding to the storage
-// precision) into e.partial[L], in FP64 and a fixed order.
-template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT = false, bool GP = false, bool TD = false, bool RED = false>
+// (dhop_site_gp).  TD: fields in the GBX_BASIS_TDIAG spin basis.  RED: also a
+// sum over the workgroup's values (RED_OUT: before their rounding to the
+// storage precision) into e.partial[L], in FP64 and a fixed order.
+template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT = false, bool GP = false, bool TD = false, int RED = RED_NONE>
 __global__ void __launch_bounds__(PF ? 256 : 1024)
     k_dhop(const void *__restrict__ gauge, const uint32_t *__restrict__ nbr, const void *__restrict__ in,
            void *__restrict__ out, const void *__restrict__ center, uint32_t nslot, uint32_t M, uint32_t spw, uint32_t mc,
@@ -318,7 +374,7 @@ __global__ void __launch_bounds__(PF ? 256 : 1024)
       m += m0;
     }
     if constexpr (EPI == EPI_S5) store_s5<P, DAG, RED>(out, center, q0 + sl, M, m, e, rr, ri, nt != 0, norm);
-    else if constexpr (RED) store_axpby_norm<P>(out, center, q0 + sl, M, m, e, rr, ri, nt != 0, norm);
+    else if constexpr (RED) store_axpby_norm<P, RED>(out, center, q0 + sl, M, m, e, rr, ri, nt != 0, norm);
     else dev::store_site<P, EPI == EPI_AXPBY>(out, center, q0 + sl, M, m, rr, ri, e.alpha, e.beta, nt != 0);
   }
   if constexpr (RED) {
@@ -345,20 +401,22 @@ struct LaunchArgs {
   const uint32_t *skip = nullptr;
   uint32_t skip_at = 0;
   double *partial = nullptr;
+  void *r = nullptr;
+  const double *a = nullptr;
 };
 
-template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT = false, bool GP = false, bool TD = false, bool RED = false>
+template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT = false, bool GP = false, bool TD = false, int RED = RED_NONE>
 void launch_t(const LaunchArgs &a)
 {
   typedef typename dev::Traits<P>::acc A;
-  const Epi<A> e{(A)a.alpha, (A)a.beta, (A)a.d, (A)a.mass, a.Ls, a.skip, a.skip_at, a.partial};
+  const Epi<A> e{(A)a.alpha, (A)a.beta, (A)a.d, (A)a.mass, a.Ls, a.skip, a.skip_at, a.partial, a.r, a.a};
   hipLaunchKernelGGL((k_dhop<P, DAG, C12, EPI, PF, EXACT, GP, TD, RED>), a.grid, a.block, a.lds, a.st, a.gauge, a.nbr, a.in,
                      a.out, a.center, a.nslot, a.M, a.spw, a.mc, a.nwg_sites, a.cblk, a.nchunk, a.nwg, a.per_xcd, a.xcd, a.nt,
                      e, a.ghost0);
 }
 
 // The fused forms (dhop_fused.hip): the fifth-dimension epilogues and the
-// forms that also sum |out|^2.
-void launch_fused(int prec, int epi, bool dag, bool c12, bool td, bool red, int pf, const LaunchArgs &a);
+// forms that also sum (RED_OUT without, RED_RESID with dag).
+void launch_fused(int prec, int epi, bool dag, bool c12, bool td, int red, int pf, const LaunchArgs &a);
 
 }  // namespace dhopk

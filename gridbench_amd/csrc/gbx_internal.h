@@ -224,9 +224,13 @@ struct dhop_fuse {
   const gbx_dwf_params *dwf = nullptr;
   const uint32_t *skip = nullptr;  // device word: nothing runs if *skip <= skip_at
   uint32_t skip_at = 0;
-  // |out|^2 of each workgroup (dag 0, with axpby or MOOEE): dhop_workgroups
-  // values.
+  // A sum of each workgroup, with axpby or MOOEE: dhop_workgroups values.  dag
+  // 0: |out|^2.  dag 1: out is not written, r -= *resid_a out is done in its
+  // place and |r|^2 summed; r has out's shape, in the arithmetic type (FP64 or
+  // FP32).
   double *partial = nullptr;
+  gbx_spinor_s *resid = nullptr;
+  const double *resid_a = nullptr;
 };
 uint32_t dhop_workgroups(const gbx_gauge_s *u, const gbx_spinor_s *in, const dhop_cfg &cfg);
 // Whether MOOEE_INV can run at this shape: one point per thread, whole columns.

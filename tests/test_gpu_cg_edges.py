@@ -69,3 +69,39 @@ def test_no_convergence_is_reported(gpu, gbx):
     assert e.value.status == 10
     gbx.cg_solve(U, Ulo, x, b, KAPPA, tol=1e-10)  # and the next solve is not disturbed
     assert residual(gbx, g, U, x, b) <= 2e-10
+
+
+# the solution is brought up to date every other iteration and when the solve
+# ends: an iteration limit at either parity must leave nothing out
+@pytest.mark.parametrize("max_inner", [1, 2, 3, 8, 9])
+@pytest.mark.parametrize("lo", [None, "f32", "bf16"])
+def test_limit_at_either_parity_follows_the_textbook_iteration(gpu, gbx, max_inner, lo):
+    dims, Ls = (4, 4, 2, 6), 3
+    g, U, Ulo, b, x = system(gbx, dims, Ls, lo)
+    with pytest.raises(gbx.GbxError):
+        gbx.cg_solve(U, Ulo, x, b, KAPPA, tol=1e-14, inner_tol=1e-13, max_outer=1, max_inner=max_inner)
+
+    t, y = (gbx.SpinorField(g, Ls, 1, "f64") for _ in range(2))
+    f = gbx.SpinorField(g, Ls, 1, "f64")
+
+    def A(v):
+        f.upload(v)
+        gbx.dhop_axpby(U, t, f, 1.0, -KAPPA)
+        gbx.dhop_axpby(U, y, t, 1.0, -KAPPA, dag=True)
+        return y.download()
+
+    r = b.download()
+    e, p, rr = np.zeros_like(r), r.copy(), np.sum(r * r)
+    for _ in range(max_inner):
+        q = A(p)
+        a = rr / np.sum(p * q)
+        e += a * p
+        r -= a * q
+        new = np.sum(r * r)
+        p = r + (new / rr) * p
+        rr = new
+    # p and t are rounded once an iteration to the inner precision (unit 2^-24,
+    # 2^-9), which moves a step by at most its condition (1 + 8 KAPPA)^2 /
+    # (1 - 8 KAPPA)^2 times that; the steps here shrink, so a few units in all
+    unit = {None: 2.0 ** -53, "f32": 2.0 ** -24, "bf16": 2.0 ** -9}[lo]
+    assert rel_l2(x.download(), e) <= max(8 * max_inner * unit, 1e-13)
