@@ -278,6 +278,7 @@ int dhop_launch(const gbx_gauge_s *u, gbx_spinor_s *out, const gbx_spinor_s *in,
   a.gauge = (const char *)u->d + q0 * 8 * (u->comp12 ? 12 : 18) * pb;
   a.nbr = u->geom->nbr + q0 * 8;
   a.in = in->d;
+  a.in_bytes = in->bytes;
   a.out = (char *)out->d + q0 * slot_bytes;
   a.center = axpby ? (const char *)center->d + q0 * slot_bytes : nullptr;
   a.xcd = c.xcd;

@@ -222,7 +222,7 @@ __device__ __forceinline__ void su3_row2(A *U)
 // into LDS as accumulation-precision 3x3 matrices [site][dir][18].
 template <int P, bool C12>
 __device__ __forceinline__ void stage_links(const void *__restrict__ gauge, const uint32_t *__restrict__ nbr, uint32_t q0,
-                                            uint32_t nsl, typename Traits<P>::acc *sU, uint32_t *sN)
+                                            uint32_t nsl, typename Traits<P>::acc *sU, uint32_t *sN, uint32_t scale = 1)
 {
   typedef typename Traits<P>::acc A;
   typedef typename Traits<P>::st S;
@@ -235,7 +235,7 @@ __device__ __forceinline__ void stage_links(const void *__restrict__ gauge, cons
     const uint32_t link = e / RL, k = e - link * RL;
     sU[link * 18 + k] = (A)__builtin_nontemporal_load(g + e);
   }
-  for (uint32_t e = threadIdx.x; e < nsl * 8; e += blockDim.x) sN[e] = nbr[(uint64_t)q0 * 8 + e];
+  for (uint32_t e = threadIdx.x; e < nsl * 8; e += blockDim.x) sN[e] = nbr[(uint64_t)q0 * 8 + e] * scale;
   if (C12) {
     __syncthreads();
     for (uint32_t l = threadIdx.x; l < nsl * 8; l += blockDim.x) su3_row2(sU + l * 18);
@@ -243,15 +243,42 @@ __device__ __forceinline__ void stage_links(const void *__restrict__ gauge, cons
   __syncthreads();
 }
 
-// Gather the 24 reals of neighbour slot `nb`, minor index m.
-template <int P>
+// Chunk k of neighbour `nb`, minor index m: `nb` is its slot, or for O32 its byte
+// offset in a field of at most 4 GiB.  The chunk's address is then a scalar base
+// (the field's, k chunks on) and a 32-bit offset, one addition a leg in place of
+// a 64-bit multiplication and an addition a load: about 100 of a point's 1000
+// VALU operations and a few registers.  The solvers' FP32 and 16-bit forms take
+// it (their hops read from the caches, where the arithmetic shows): CG at
+// 16^3x24 x Ls8, FP16 inner, 11.72 -> 11.33 ms, domain-wall solve 16^4 x Ls12,
+// FP32 inner, 15.08 -> 14.76 ms.  The others are bound by the L2 misses and run
+// no faster or up to 1.6 % slower (24^4 x Ls16 FP64 748 -> 760 us; BF16 16^3x24
+// x Ls12 x 16 704 either way), as their gathers then come in denser bursts.
+template <int P, bool O32>
+__device__ __forceinline__ typename Traits<P>::vec load_at(const void *__restrict__ in, uint32_t nb, uint32_t M, uint32_t m, int k)
+{
+  typedef typename Traits<P>::vec V;
+  if constexpr (O32) {
+    typedef const __attribute__((address_space(1))) char *G;
+    G base = (G)in + (uint64_t)k * M * 16;
+    asm("" : "+s"(base));  // kept apart from the offset
+    return *(const __attribute__((address_space(1))) V *)(base + (nb + m * 16));
+  } else {
+    return ((const V *)in)[(uint64_t)nb * Traits<P>::NCH * M + m + (uint64_t)k * M];
+  }
+}
+
+// Gather the 24 reals of a neighbour.
+template <int P, bool O32 = false>
 __device__ __forceinline__ void load_nb(const void *__restrict__ in, uint32_t nb, uint32_t M, uint32_t m,
                                         typename Traits<P>::acc *v)
 {
   constexpr int NCH = Traits<P>::NCH, R = Traits<P>::R;
-  const uint64_t base = (uint64_t)nb * NCH * M + m;
 #pragma unroll
-  for (int k = 0; k < NCH; k++) load_chunk<P, typename Traits<P>::acc>(in, base + (uint64_t)k * M, v + k * R);
+  for (int k = 0; k < NCH; k++) {
+    const typename Traits<P>::vec x = load_at<P, O32>(in, nb, M, m, k);
+#pragma unroll
+    for (int j = 0; j < R; j++) v[k * R + j] = (typename Traits<P>::acc)x[j];
+  }
 }
 
 // project, multiply by U (18 reals in LDS), reconstruct into r
@@ -317,15 +344,17 @@ template <bool DAG, int D, bool TD> struct LegHalf {
 };
 
 // Chunks of one spin half (v[0..11] = its 2 spins x 3 colours).
-template <int P, bool UPPER>
+template <int P, bool UPPER, bool O32 = false>
 __device__ __forceinline__ void load_nb_half(const void *__restrict__ in, uint32_t nb, uint32_t M, uint32_t m,
                                              typename Traits<P>::acc *v)
 {
   constexpr int NCH = Traits<P>::NCH, R = Traits<P>::R, K0 = UPPER ? 0 : NCH / 2;
-  const uint64_t base = (uint64_t)nb * NCH * M + m;
 #pragma unroll
-  for (int k = 0; k < NCH / 2; k++)
-    load_chunk<P, typename Traits<P>::acc>(in, base + (uint64_t)(K0 + k) * M, v + k * R);
+  for (int k = 0; k < NCH / 2; k++) {
+    const typename Traits<P>::vec x = load_at<P, O32>(in, nb, M, m, K0 + k);
+#pragma unroll
+    for (int j = 0; j < R; j++) v[k * R + j] = (typename Traits<P>::acc)x[j];
+  }
 }
 
 template <bool UPPER, int MUL, typename A>
@@ -346,12 +375,12 @@ __device__ __forceinline__ void leg_half(const A *v, const A *U, A *rr, A *ri)
   }
 }
 
-template <int P, bool DAG, int D, bool TD>
+template <int P, bool DAG, int D, bool TD, bool O32 = false>
 __device__ __forceinline__ void leg_load(const void *__restrict__ in, uint32_t nb, uint32_t M, uint32_t m,
                                          typename Traits<P>::acc *v)
 {
-  if constexpr (LegHalf<DAG, D, TD>::value) load_nb_half<P, LegHalf<DAG, D, TD>::upper>(in, nb, M, m, v);
-  else load_nb<P>(in, nb, M, m, v);
+  if constexpr (LegHalf<DAG, D, TD>::value) load_nb_half<P, LegHalf<DAG, D, TD>::upper, O32>(in, nb, M, m, v);
+  else load_nb<P, O32>(in, nb, M, m, v);
 }
 
 // The leg arithmetic runs at raised wave priority (s_setprio 1), the gathers
@@ -388,12 +417,11 @@ __device__ __forceinline__ void pin_acc(A *rr, A *ri)
 // unchained products, took 1250 operations a point (190 of 243 us); 880 here,
 // 211 us.  BF16 keeps its conversions: 1075.  16^3x24 x Ls12 x 16 BF16: 777 ->
 // 659 us.
-template <int P>
+template <int P, bool O32 = false>
 __device__ __forceinline__ void load_raw(const void *__restrict__ in, uint32_t nb, uint32_t M, uint32_t m, RawReals<P> &v)
 {
-  const typename Traits<P>::vec *p = (const typename Traits<P>::vec *)in + (uint64_t)nb * Traits<P>::NCH * M + m;
 #pragma unroll
-  for (int k = 0; k < Traits<P>::NCH; k++) v.c[k] = p[(uint64_t)k * M];
+  for (int k = 0; k < Traits<P>::NCH; k++) v.c[k] = load_at<P, O32>(in, nb, M, m, k);
 }
 
 template <int P, bool DAG, int D>
@@ -410,7 +438,7 @@ __device__ __forceinline__ void leg_raw(const RawReals<P> &v, const float *U, fl
 // PF legs are gathered ahead of the one being computed; the scheduling barrier
 // and the pinned accumulators keep the compiler from gathering (and holding)
 // more of them, or from sinking the arithmetic into the stores' branches.
-template <int P, bool DAG, int PF>
+template <int P, bool DAG, int PF, bool O32>
 __device__ __forceinline__ void dhop_site_raw(const void *__restrict__ in, const uint32_t *nb, uint32_t M, uint32_t m,
                                               const float *U, float *rr, float *ri)
 {
@@ -420,9 +448,9 @@ __device__ __forceinline__ void dhop_site_raw(const void *__restrict__ in, const
 #pragma unroll
   for (int d = 0; d <= PF; d++) v[d].one = one;
 #pragma unroll
-  for (int d = 0; d < PF; d++) load_raw<P>(in, nb[d], M, m, v[d]);
+  for (int d = 0; d < PF; d++) load_raw<P, O32>(in, nb[d], M, m, v[d]);
 #define GBX_RLEG(D)                                                                \
-  if (D + PF < 8) load_raw<P>(in, nb[(D + PF) & 7], M, m, v[(D + PF) % (PF + 1)]); \
+  if (D + PF < 8) load_raw<P, O32>(in, nb[(D + PF) & 7], M, m, v[(D + PF) % (PF + 1)]); \
   __builtin_amdgcn_sched_barrier(0);                                               \
   leg_raw<P, DAG, D>(v[D % (PF + 1)], U + D * 18, rr, ri);                         \
   pin_acc(rr, ri);                                                                 \
@@ -444,7 +472,7 @@ __device__ __forceinline__ void dhop_site_raw(const void *__restrict__ in, const
 // keeps a second set of loads in flight per wavefront.  PF = 2: three
 // buffers, gathers two legs ahead.  EXACT: the reference's rounding in the
 // SU(3) products (FP64 / FP32).  TD: GBX_BASIS_TDIAG fields (LegKind, LegHalf).
-template <int P, bool DAG, int PF, bool EXACT = false, bool TD = false>
+template <int P, bool DAG, int PF, bool EXACT = false, bool TD = false, bool O32 = false>
 __device__ __forceinline__ void dhop_site(const void *__restrict__ in, const uint32_t *nb, uint32_t M, uint32_t m,
                                           const typename Traits<P>::acc *U, typename Traits<P>::acc *rr,
                                           typename Traits<P>::acc *ri)
@@ -453,11 +481,11 @@ __device__ __forceinline__ void dhop_site(const void *__restrict__ in, const uin
   constexpr int CH = EXACT ? MUL_EXACT : MUL_CHAIN;
   if constexpr (P == GBX_F16 || P == GBX_BF16) {
     static_assert(!EXACT && !TD, "FP64 / FP32 forms");
-    dhop_site_raw<P, DAG, PF>(in, nb, M, m, U, rr, ri);
+    dhop_site_raw<P, DAG, PF, O32>(in, nb, M, m, U, rr, ri);
   } else if (PF == 0) {
     A v[24];
 #define GBX_LEG(D, FIRST)                                                  \
-    leg_load<P, DAG, D, TD>(in, nb[D], M, m, v);                           \
+    leg_load<P, DAG, D, TD, O32>(in, nb[D], M, m, v);                           \
     leg_apply<DAG, D, TD, FIRST, CH>(v, U + D * 18, rr, ri);
     GBX_LEG(0, true)
     GBX_LEG(1, false)
@@ -470,38 +498,38 @@ __device__ __forceinline__ void dhop_site(const void *__restrict__ in, const uin
 #undef GBX_LEG
   } else if (PF == 2) {
     A v0[24], v1[24], v2[24];
-    leg_load<P, DAG, 0, TD>(in, nb[0], M, m, v0);
-    leg_load<P, DAG, 1, TD>(in, nb[1], M, m, v1);
-    leg_load<P, DAG, 2, TD>(in, nb[2], M, m, v2);
+    leg_load<P, DAG, 0, TD, O32>(in, nb[0], M, m, v0);
+    leg_load<P, DAG, 1, TD, O32>(in, nb[1], M, m, v1);
+    leg_load<P, DAG, 2, TD, O32>(in, nb[2], M, m, v2);
     leg_apply<DAG, 0, TD, true, CH>(v0, U + 0 * 18, rr, ri);
-    leg_load<P, DAG, 3, TD>(in, nb[3], M, m, v0);
+    leg_load<P, DAG, 3, TD, O32>(in, nb[3], M, m, v0);
     leg_apply<DAG, 1, TD, false, CH>(v1, U + 1 * 18, rr, ri);
-    leg_load<P, DAG, 4, TD>(in, nb[4], M, m, v1);
+    leg_load<P, DAG, 4, TD, O32>(in, nb[4], M, m, v1);
     leg_apply<DAG, 2, TD, false, CH>(v2, U + 2 * 18, rr, ri);
-    leg_load<P, DAG, 5, TD>(in, nb[5], M, m, v2);
+    leg_load<P, DAG, 5, TD, O32>(in, nb[5], M, m, v2);
     leg_apply<DAG, 3, TD, false, CH>(v0, U + 3 * 18, rr, ri);
-    leg_load<P, DAG, 6, TD>(in, nb[6], M, m, v0);
+    leg_load<P, DAG, 6, TD, O32>(in, nb[6], M, m, v0);
     leg_apply<DAG, 4, TD, false, CH>(v1, U + 4 * 18, rr, ri);
-    leg_load<P, DAG, 7, TD>(in, nb[7], M, m, v1);
+    leg_load<P, DAG, 7, TD, O32>(in, nb[7], M, m, v1);
     leg_apply<DAG, 5, TD, false, CH>(v2, U + 5 * 18, rr, ri);
     leg_apply<DAG, 6, TD, false, CH>(v0, U + 6 * 18, rr, ri);
     leg_apply<DAG, 7, TD, false, CH>(v1, U + 7 * 18, rr, ri);
   } else {
     A v0[24], v1[24];
-    leg_load<P, DAG, 0, TD>(in, nb[0], M, m, v0);
-    leg_load<P, DAG, 1, TD>(in, nb[1], M, m, v1);
+    leg_load<P, DAG, 0, TD, O32>(in, nb[0], M, m, v0);
+    leg_load<P, DAG, 1, TD, O32>(in, nb[1], M, m, v1);
     leg_apply<DAG, 0, TD, true, CH>(v0, U + 0 * 18, rr, ri);
-    leg_load<P, DAG, 2, TD>(in, nb[2], M, m, v0);
+    leg_load<P, DAG, 2, TD, O32>(in, nb[2], M, m, v0);
     leg_apply<DAG, 1, TD, false, CH>(v1, U + 1 * 18, rr, ri);
-    leg_load<P, DAG, 3, TD>(in, nb[3], M, m, v1);
+    leg_load<P, DAG, 3, TD, O32>(in, nb[3], M, m, v1);
     leg_apply<DAG, 2, TD, false, CH>(v0, U + 2 * 18, rr, ri);
-    leg_load<P, DAG, 4, TD>(in, nb[4], M, m, v0);
+    leg_load<P, DAG, 4, TD, O32>(in, nb[4], M, m, v0);
     leg_apply<DAG, 3, TD, false, CH>(v1, U + 3 * 18, rr, ri);
-    leg_load<P, DAG, 5, TD>(in, nb[5], M, m, v1);
+    leg_load<P, DAG, 5, TD, O32>(in, nb[5], M, m, v1);
     leg_apply<DAG, 4, TD, false, CH>(v0, U + 4 * 18, rr, ri);
-    leg_load<P, DAG, 6, TD>(in, nb[6], M, m, v0);
+    leg_load<P, DAG, 6, TD, O32>(in, nb[6], M, m, v0);
     leg_apply<DAG, 5, TD, false, CH>(v1, U + 5 * 18, rr, ri);
-    leg_load<P, DAG, 7, TD>(in, nb[7], M, m, v1);
+    leg_load<P, DAG, 7, TD, O32>(in, nb[7], M, m, v1);
     leg_apply<DAG, 6, TD, false, CH>(v0, U + 6 * 18, rr, ri);
     leg_apply<DAG, 7, TD, false, CH>(v1, U + 7 * 18, rr, ri);
   }

@@ -307,8 +307,9 @@ __device__ __forceinline__ double block_sum(double a)
 // GP: a domain part whose ghosts hold spin-projected halves from ghost0 on
 // (dhop_site_gp).  TD: fields in the GBX_BASIS_TDIAG spin basis.  RED: also a
 // sum over the workgroup's values (RED_OUT: before their rounding to the
-// storage precision) into e.partial[L], in FP64 and a fixed order.
-template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT = false, bool GP = false, bool TD = false, int RED = RED_NONE>
+// storage precision) into e.partial[L], in FP64 and a fixed order.  O32: 32-bit
+// gather offsets (dev::load_at).
+template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT, bool GP, bool TD, int RED, bool O32>
 __global__ void __launch_bounds__(PF ? 256 : 1024)
     k_dhop(const void *__restrict__ gauge, const uint32_t *__restrict__ nbr, const void *__restrict__ in,
            void *__restrict__ out, const void *__restrict__ center, uint32_t nslot, uint32_t M, uint32_t spw, uint32_t mc,
@@ -336,7 +337,7 @@ __global__ void __launch_bounds__(PF ? 256 : 1024)
   }
   const uint32_t q0 = b * spw, m0 = chunk * mc;
   const uint32_t nsl = min(spw, nslot - q0), mcc = min(mc, M - m0);
-  dev::stage_links<P, C12>(gauge, nbr, q0, nsl, sU, sN);
+  dev::stage_links<P, C12>(gauge, nbr, q0, nsl, sU, sN, O32 ? dev::Traits<P>::NCH * M * 16 : 1);
 
   const uint32_t items = nsl * mcc;
   if constexpr (EPI == EPI_S5INV || EPI == EPI_S5X) {  // one point per thread, whole columns
@@ -344,7 +345,7 @@ __global__ void __launch_bounds__(PF ? 256 : 1024)
     const bool active = w < items;
     A rr[12], ri[12];
     if (active) {
-      dev::dhop_site<P, DAG, PF, EXACT, TD>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
+      dev::dhop_site<P, DAG, PF, EXACT, TD, O32>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
       dev::pin_acc(rr, ri);
     }
     again(w, mcc, sl, m);
@@ -366,7 +367,7 @@ __global__ void __launch_bounds__(PF ? 256 : 1024)
     uint32_t sl = w / mcc, m = m0 + (w - sl * mcc);
     A rr[12], ri[12];
     if constexpr (GP) dev::dhop_site_gp<P, DAG, PF>(in, sN + sl * 8, M, m, ghost0, sU + sl * 8 * 18, rr, ri);
-    else dev::dhop_site<P, DAG, PF, EXACT, TD>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
+    else dev::dhop_site<P, DAG, PF, EXACT, TD, O32>(in, sN + sl * 8, M, m, sU + sl * 8 * 18, rr, ri);
     if constexpr (EPI == EPI_AXPBY && RED) {
       uint32_t w2 = w;
       dev::pin_acc(rr, ri);
@@ -403,6 +404,7 @@ struct LaunchArgs {
   double *partial = nullptr;
   void *r = nullptr;
   const double *a = nullptr;
+  uint64_t in_bytes = 0;
 };
 
 template <int P, bool DAG, bool C12, int EPI, int PF, bool EXACT = false, bool GP = false, bool TD = false, int RED = RED_NONE>
@@ -410,9 +412,12 @@ void launch_t(const LaunchArgs &a)
 {
   typedef typename dev::Traits<P>::acc A;
   const Epi<A> e{(A)a.alpha, (A)a.beta, (A)a.d, (A)a.mass, a.Ls, a.skip, a.skip_at, a.partial, a.r, a.a};
-  hipLaunchKernelGGL((k_dhop<P, DAG, C12, EPI, PF, EXACT, GP, TD, RED>), a.grid, a.block, a.lds, a.st, a.gauge, a.nbr, a.in,
-                     a.out, a.center, a.nslot, a.M, a.spw, a.mc, a.nwg_sites, a.cblk, a.nchunk, a.nwg, a.per_xcd, a.xcd, a.nt,
-                     e, a.ghost0);
+  auto *k = &k_dhop<P, DAG, C12, EPI, PF, EXACT, GP, TD, RED, false>;
+  if constexpr (P != GBX_F64 && (EPI >= EPI_S5 || RED != RED_NONE)) {
+    if (a.in_bytes <= (1ull << 32)) k = &k_dhop<P, DAG, C12, EPI, PF, EXACT, GP, TD, RED, true>;
+  }
+  hipLaunchKernelGGL(k, a.grid, a.block, a.lds, a.st, a.gauge, a.nbr, a.in, a.out, a.center, a.nslot, a.M, a.spw, a.mc,
+                     a.nwg_sites, a.cblk, a.nchunk, a.nwg, a.per_xcd, a.xcd, a.nt, e, a.ghost0);
 }
 
 // The fused forms (dhop_fused.hip): the fifth-dimension epilogues and the
