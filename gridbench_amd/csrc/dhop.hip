@@ -120,9 +120,8 @@ bool dhop_lookup_cfg(const std::string &sig, gbx_kcfg *c)
 
 // The shape of a problem nobody tuned: a rule fitted to 300 shapes (extents
 // 4..24, Ls 4..20, 1..16 right-hand sides, whole lattices and red-black
-// halves), each timed in 30 configurations: on fresh shapes it is 2.4 % slower
-// than the best of the 30 on average (25 % at worst); one workgroup of 256 or
-// more threads without the pipeline, whatever the size, was 18 % (89 %).
+// halves), each timed in 30 configurations; on 180 fresh shapes it is 1.9 %
+// slower than the best of up to 50 on average (13 % at worst).
 //  * mc: above 88 minor indices (16-bit: 128) a workgroup takes chunks of
 //    40..88 of them, whole 128-byte lines, the size that leaves the fewest
 //    lanes idle: a smaller set of neighbours in flight, which the L2s hold
@@ -132,9 +131,10 @@ bool dhop_lookup_cfg(const std::string &sig, gbx_kcfg *c)
 //    points (more workgroups, no barrier between wavefronts), 256 threads
 //    otherwise, where the links of more sites are staged together; with one
 //    or two sites in a wavefront, a larger workgroup if it idles fewer lanes.
-//  * pf: the gather pipeline pays for its registers (FP64 2 wavefronts a SIMD
-//    instead of 4, FP32 5 instead of 8, 16-bit 6 instead of 7 or 8) except
-//    where the whole grid is resident in one round without it and not with it.
+//  * pf: one leg ahead, or two where a chunk of more than 64 FP64 / FP32 minor
+//    indices fills the wavefronts (FP32: 4.2 instead of 7.4 % from the best).
+//    Without the pipeline every precision is 11 to 14 % from the best, also
+//    where the registers it saves would hold the whole grid in one round.
 dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
 {
   const bool f64 = in->prec == GBX_F64, f32 = in->prec == GBX_F32, f16 = !f64 && !f32;
@@ -166,16 +166,13 @@ dhop_cfg dhop_default_cfg(const gbx_gauge_s *u, const gbx_spinor_s *in)
     while (threads < 256 && sites(threads, M) * M * 5 < threads * 3) threads += 64;  // 3/5 of the lanes busy
     spw = sites(threads, M);
   }
-  const uint64_t waves = (vol + spw - 1) / spw * ((M + mc - 1) / mc) * (threads / 64);
   dhop_cfg c;
   c.spw = (int)spw;
   c.threads = (int)threads;
   c.xcd = 1;
   c.nt = 1;
   c.mc = mc == M ? 0 : (int)mc;
-  if (f64) c.pf = waves > 2048 && waves <= (M < 16 ? 3584u : 3072u) ? 0 : M <= 24 ? 1 : 2;
-  else if (f32) c.pf = M <= 16 && waves > 5120 && waves <= 8192 ? 0 : M <= 24 ? 1 : 2;
-  else c.pf = M <= 64 && waves > 6144 && waves <= (in->prec == GBX_F16 ? 8192u : 7168u) ? 0 : 1;
+  c.pf = f16 || M <= 64 ? 1 : 2;
   c.axpby_pf = true;
   c.wgpc = 0;
   c.cblk = 0;

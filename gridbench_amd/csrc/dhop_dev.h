@@ -220,22 +220,60 @@ __device__ __forceinline__ void su3_row2(A *U)
 
 // Stage the links (and neighbour slots) of workgroup sites q0 .. q0+nsl-1
 // into LDS as accumulation-precision 3x3 matrices [site][dir][18].
+// A workgroup can gather nothing before this is done, so it should cost one
+// memory round trip: the neighbour slots and up to N 16-byte pieces of links a
+// thread are all loaded before the first is stored to LDS (N covers a default
+// shape with minor extents from 6 on).  One real at a time, each waited for, it
+// was 9 round trips in FP64 at Ls 16 and 18 at Ls 8: FP64 8^4 x Ls8 6.8 -> 4.8
+// us; FP32 20x18x10x14 x Ls10 37.2 -> 36.0 us; FP64 24^4 x Ls16 747 -> 735 us;
+// CG at 16^3x24 x Ls8, FP16 inner, 11.7 -> 9.6 ms, domain-wall solve 16^4 x
+// Ls12, FP32 inner, 15.2 -> 13.5 ms.  With many right-hand sides, where a
+// workgroup's staging was short before, it is level or 1 % behind (FP32 16^4 x
+// Ls16 x 8: 597 -> 605 us).
 template <int P, bool C12>
 __device__ __forceinline__ void stage_links(const void *__restrict__ gauge, const uint32_t *__restrict__ nbr, uint32_t q0,
                                             uint32_t nsl, typename Traits<P>::acc *sU, uint32_t *sN, uint32_t scale = 1)
 {
   typedef typename Traits<P>::acc A;
   typedef typename Traits<P>::st S;
-  constexpr int RL = C12 ? 12 : 18;
-  const S *g = (const S *)gauge + (uint64_t)q0 * 8 * RL;
-  const uint32_t n = nsl * 8 * RL;
-  // Links are read once per launch: non-temporal loads keep them from
-  // displacing neighbour spinors, which are re-read, in the L2.
-  for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) {
-    const uint32_t link = e / RL, k = e - link * RL;
-    sU[link * 18 + k] = (A)__builtin_nontemporal_load(g + e);
+  typedef typename Traits<P>::vec V;
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  constexpr int RL = C12 ? 12 : 18, R = Traits<P>::R, PS = 8 * RL / R;  // pieces of a site
+  constexpr int N = P == GBX_F64 ? 12 : P == GBX_F32 ? 8 : 4;
+  const V *g = (const V *)((const S *)gauge + (uint64_t)q0 * 8 * RL);
+  const u4 *gn = (const u4 *)(nbr + (uint64_t)q0 * 8);
+  const uint32_t n = nsl * PS, nn = nsl * 2, th = blockDim.x;
+  u4 nb;
+  if (threadIdx.x < nn) nb = gn[threadIdx.x];
+  for (uint32_t e0 = threadIdx.x; e0 < n; e0 += N * th) {
+    V x[N];
+    // Links are read once per launch: non-temporal loads keep them from
+    // displacing neighbour spinors, which are re-read, in the L2.
+#pragma unroll
+    for (int i = 0; i < N; i++)
+      if (e0 + i * th < n) x[i] = __builtin_nontemporal_load(g + e0 + i * th);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const uint32_t e = e0 + i * th;
+      if (e >= n) break;
+      if constexpr (!C12 && R * sizeof(A) == 16) {
+        ((V *)sU)[e] = x[i];
+      } else {
+#pragma unroll
+        for (int j = 0; j < R; j += 2) {  // a link's reals are even in number
+          const uint32_t r = e * R + j, link = r / RL;
+          A *d = sU + link * (18 - RL) + r;
+          d[0] = (A)x[i][j];
+          d[1] = (A)x[i][j + 1];
+        }
+      }
+    }
   }
-  for (uint32_t e = threadIdx.x; e < nsl * 8; e += blockDim.x) sN[e] = nbr[(uint64_t)q0 * 8 + e] * scale;
+  for (uint32_t e = threadIdx.x; e < nn; e += th) {
+    if (e != threadIdx.x) nb = gn[e];
+    ((u4 *)sN)[e] = nb * scale;
+  }
   if (C12) {
     __syncthreads();
     for (uint32_t l = threadIdx.x; l < nsl * 8; l += blockDim.x) su3_row2(sU + l * 18);
