@@ -24,13 +24,14 @@
 // The scalars stay on the device, so no kernel waits for the host.  The host
 // enqueues a few iterations ahead and learns of convergence from a word the
 // device writes to its memory; what was enqueued beyond it does nothing.
-// An iteration at 16^3x24 x Ls8, FP16 inner, takes 137 us with no gaps: 42 us
-// for M p, 55 us for M^dag t with the update of r, 5 us for k_cg_alpha, and 23
-// or 45 us for k_cg_ep (6 TB/s).  It took 307 us with the two sums read back by
+// An iteration at 16^3x24 x Ls8, FP16 inner, takes 111 us with no gaps: 33 us
+// for M p, 39 us for M^dag t with the update of r, 5 us for k_cg_alpha, and 23
+// or 46 us for k_cg_ep (6 TB/s).  It took 307 us with the two sums read back by
 // the host and the updates in passes of their own, and 163 us with the scalars
 // on the device but M^dag t stored and read again (30 us) and e updated each
-// time (42 us): 13.6 -> 12.0 ms a solve; domain-wall solve 16^4 x Ls12, FP32
-// inner: 16.3 -> 15.2 ms.  The partial sums are summed where they are needed
+// time (42 us): 13.6 -> 12.0 ms a solve (9.7 since the hops stage their links
+// in one round trip); domain-wall solve 16^4 x Ls12, FP32 inner: 16.3 -> 15.2
+// ms (13.5).  The partial sums are summed where they are needed
 // up to kPlain of them, which costs a reader 2 us; a pass of its own takes 5.
 #include <algorithm>
 #include <chrono>

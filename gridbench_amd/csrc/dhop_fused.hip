@@ -5,7 +5,7 @@
 // The hopping kernels are bound by their gathers (dhop.hip), so what an
 // epilogue adds is the traffic of its own operands: D = Mooee - Dhop / 2 at
 // 24^4 x Ls16 FP64 took 836 us for Dhop and 491 us for a pass over three
-// fields that adds Mooee; in one kernel it takes 863 us (FP32: 627 -> 424 us),
+// fields that adds Mooee; in one kernel it takes 857 us (FP32: 627 -> 424 us),
 // 50 us over Dhop alone for a third field to read.  The even-odd operator's
 // Mooee^-1 DhopOE (16^4 x Ls12 FP32: 29 + 16 us as two kernels) saves the pass
 // over the half lattice too; the domain-wall solve there went from 26.4 to
